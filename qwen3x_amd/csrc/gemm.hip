@@ -6,6 +6,7 @@
 // path is an FP32 SIMT kernel (batch_mv_q8_kernel :761, 64 rows x 128 tokens
 // per CTA) and which has no Q4_0 GEMM (it asserts, :1580).
 #include "gemm.h"
+#include "gemm_thin.h"
 #include "gemm_x3.h"
 #include "matvec.h"
 
@@ -71,6 +72,13 @@ int gemm(const void* w, uint32_t type, int rows, int cols, const float* X, int c
             if (status != Q3X_HIP_OK) return status;
         }
         return Q3X_HIP_OK;
+    }
+    // A few tokens: the launch that reads the weights once, in whole row
+    // segments (launch_thin).
+    if (thin_ok(count, cols, aligned(w, 16))) {
+        DenseGemm t{0, X, cols, count, static_cast<const uint8_t*>(w), row_bytes, Y, rows, accumulate != 0};
+        return type == Q3X_HIP_MATRIX_Q8_0 ? launch_thin<Q3X_HIP_MATRIX_Q8_0>(t, rows, count, cols, stream)
+                                           : launch_thin<Q3X_HIP_MATRIX_Q4_0>(t, rows, count, cols, stream);
     }
     // The split plan runs only with all of the workspace it asks for (16-byte
     // aligned); otherwise q3x_hip_gemm's plan.

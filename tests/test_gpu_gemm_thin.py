@@ -1,0 +1,69 @@
+"""GPU tests of the few-token GEMM (at most 32 tokens): every tile height and
+its edges, row counts around the 16-row tiles and around the row tiles per
+workgroup, rows shorter than the waves' K units, both formats.  Each output
+against W x in float64 within the bound of the GEMM tests (1e-5 ||w|| ||x||),
+and against the general tiles (reached through a matrix that is not 16-byte
+aligned) within the two paths' FP32 rounding."""
+import numpy as np
+import pytest
+
+import qwen3x_amd as q3x
+from tests.helpers import Q4_0, Q8_0, dequant_numpy, random_blocks, row_bound
+from tests.test_gpu_parity import _torch, dev, host, say
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(type_, w, rows, cols, X, offset, add):
+    torch = _torch()
+    buf = torch.zeros(offset + w.size + 64, dtype=torch.uint8, device="cuda:0")
+    buf[offset:offset + w.size] = dev(w.reshape(-1))
+    T = X.shape[0]
+    out = torch.full((T * rows + 8,), 3.0, dtype=torch.float32, device="cuda:0")
+    q3x.batch_mv(q3x.Linear(buf[offset:offset + w.size], rows, cols, type_), dev(X), out, T, add=add)
+    got = host(out)
+    assert np.all(got[T * rows:] == 3.0), "wrote past the output"
+    return got[:T * rows].reshape(T, rows).astype(np.float64) - (3.0 if add else 0.0)
+
+
+@pytest.mark.parametrize("type_", [Q8_0, Q4_0])
+@pytest.mark.parametrize("tokens", [1, 4, 5, 8, 9, 16, 17, 32, 33])
+@pytest.mark.parametrize("rows,cols", [(1, 256), (15, 512), (49, 2304), (33, 4096), (4097, 1024), (8200, 256),
+                                       (12300, 256)])
+def test_few_token_gemm(type_, tokens, rows, cols):
+    rng = np.random.default_rng(type_ + tokens * 64 + rows)
+    w = random_blocks(rng, type_, rows, cols)
+    X = rng.normal(0, 1, (tokens, cols)).astype(np.float32)
+    wd = dequant_numpy(w, type_, rows, cols).astype(np.float64)
+    want = X.astype(np.float64) @ wd.T
+    bound = np.stack([row_bound(wd, x) for x in X])
+    say(f"few-token gemm type={type_} {tokens}x{rows}x{cols}")
+    got = _run(type_, w, rows, cols, X, 0, False)
+    assert np.all(np.abs(got - want) <= bound)
+    # Reading 3 back after adding costs up to half an ulp of the sum.
+    added = _run(type_, w, rows, cols, X, 0, True)
+    assert np.all(np.abs(added - want) <= bound + 2.0 ** -23 * (3.0 + np.abs(want)))
+    general = _run(type_, w, rows, cols, X, 2, False)
+    # Two FP32 sums of the same exact products: at most 2 (K + 40) 2^-24 of
+    # the sum of their magnitudes, far below the bound above.
+    scale = np.abs(X).astype(np.float64) @ np.abs(wd).T
+    assert np.all(np.abs(got - general) <= 2 * (cols + 40) * 2.0 ** -24 * scale)
+
+
+@pytest.mark.parametrize("type_", [Q8_0, Q4_0])
+@pytest.mark.parametrize("tokens", [3, 7, 16])
+def test_few_token_gemm_keeps_tokens_apart(type_, tokens):
+    """An infinite activation reaches its own token's outputs only, in every
+    row group that shares operand registers."""
+    rows, cols = 64, 1024
+    rng = np.random.default_rng(tokens)
+    w = random_blocks(rng, type_, rows, cols)
+    X = rng.normal(0, 1, (tokens, cols)).astype(np.float32)
+    clean = _run(type_, w, rows, cols, X, 0, False)
+    for col in (0, 33, 64, 100, 1023):
+        bad = X.copy()
+        bad[1, col] = np.inf
+        got = _run(type_, w, rows, cols, bad, 0, False)
+        keep = [t for t in range(tokens) if t != 1]
+        assert np.array_equal(got[keep], clean[keep])
+        assert not np.isfinite(got[1]).all()
