@@ -9,61 +9,57 @@
 namespace q3x {
 
 // A unit of weights: 16 consecutive rows of one K segment of BLOCKS blocks,
-// held as 144 bytes a row (Q8_0: 4 blocks are 136 bytes and the load takes 8
-// more; Q4_0: 8 blocks).  2304 bytes: two 16-byte loads a lane and one of 4.
-template <uint32_t QT>
+// PITCH bytes a row in LDS, loaded as 16-byte words a lane and one last dword.
+// ANY = false: rows of whole units, every row piece 16-byte aligned.  Q8_0: 4
+// blocks are 136 bytes and the load takes 8 more; Q4_0: 8 blocks, 144 bytes.
+// ANY = true: rows of any number of blocks (the last unit may be short), 2-byte
+// aligned; a row piece is loaded from the dword at or before its start, so a
+// row of odd number starts 2 bytes in where a row is not whole dwords.
+template <uint32_t QT, bool ANY>
 struct SegUnit {
     static constexpr bool kQ4 = QT == Q3X_HIP_MATRIX_Q4_0;
     static constexpr int BB = kQ4 ? kQ4Bytes : kQ8Bytes;
-    static constexpr int BLOCKS = kQ4 ? 8 : 4;
-    static constexpr int STEP = BLOCKS * BB;  // bytes from a segment to the row's next
-    static constexpr int PITCH = 144;
+    static constexpr int BLOCKS = kQ4 && !ANY ? 8 : 4;
+    static constexpr int STEP = BLOCKS * BB;  // bytes from a segment to the row's next: whole dwords
+    static constexpr int PITCH = kQ4 && ANY ? 80 : 144;
     static constexpr int BYTES = 16 * PITCH;
     static constexpr int WIDE = BYTES / 1024;
-    static_assert(BYTES == WIDE * 1024 + 256 && STEP <= PITCH, "two 16-byte loads a lane and one of 4 bytes");
+    static_assert(BYTES == WIDE * 1024 + 256 && STEP + (ANY ? 2 : 0) <= PITCH && STEP % 4 == 0,
+                  "16-byte words and one dword a lane hold the row pieces");
 };
 
+template <int WIDE>
 struct SegRegs {
-    u32x4 wide[2];
+    u32x4 wide[WIDE];
     uint32_t rest;
 };
 
-// This lane's bf16 operand of block kb of a unit in LDS -- weight row l16,
-// the eight values of chunk g16 -- and the row's block scale.  Q8_0: elements
-// 8 g16 + [0, 8).  Q4_0: elements 4 g16 + [0, 4) and 16 + 4 g16 + [0, 4), as
-// 16 (n - 8) with the scale d / 16 (BlockPart::values).
-template <uint32_t QT>
-__device__ __forceinline__ bf16x8 seg_operand(const uint8_t* unit, int l16, int g16, int kb, float& d) {
-    using U = SegUnit<QT>;
-    const uint8_t* blk = unit + l16 * U::PITCH + kb * U::BB;
-    const uint32_t half = *reinterpret_cast<const uint16_t*>(blk);
-    d = U::kQ4 ? f16_fast(half) * 0.0625f : f16_fast(half);
-    asm("" : "+v"(d));  // an FP32 value: v_fma_f32 issues at twice v_fma_mix_f32's rate
+// This lane's bf16 operand of block kb of a unit in LDS: weight row l16, the
+// eight values of chunk g16.  Q8_0: elements 8 g16 + [0, 8).  Q4_0: elements
+// 4 g16 + [0, 4) and 16 + 4 g16 + [0, 4), as 16 (n - 8) (BlockPart::values;
+// the scale is then d / 16).  skew: bytes the row starts late by (ANY).
+template <uint32_t QT, bool ANY>
+__device__ __forceinline__ bf16x8 seg_operand(const uint8_t* unit, int l16, int g16, int kb, int skew) {
+    using U = SegUnit<QT, ANY>;
+    const uint8_t* values = unit + l16 * U::PITCH + kb * U::BB + 2 + (U::kQ4 ? 4 : 8) * g16;
+    // Whole dwords around them; aligned rows start 2 bytes into one for even
+    // kb, on one for odd.
+    const int late = ANY ? (2 * (kb + 1) + skew) % 4 : 2 * ((kb + 1) % 2);
+    const uint32_t* a = reinterpret_cast<const uint32_t*>(values + (ANY ? skew : 0) - late);
     float v[8];
-    // A block's values start 2 bytes past a dword for even kb, on one for odd.
     if constexpr (U::kQ4) {
-        uint32_t w;
-        if (kb % 2) {
-            w = *reinterpret_cast<const uint32_t*>(blk + 2 + 4 * g16);
-        } else {
-            const uint32_t* a = reinterpret_cast<const uint32_t*>(blk + 4 * g16);
-            w = __builtin_amdgcn_alignbyte(a[1], a[0], 2);
-        }
+        const uint32_t w = ANY || late ? __builtin_amdgcn_alignbyte(a[1], a[0], late) : a[0];
         const uint32_t lo = ((w << 4) ^ 0x80808080u) & 0xf0f0f0f0u;
         const uint32_t hi = (w ^ 0x80808080u) & 0xf0f0f0f0u;
         v[0] = sbyte<0>(lo); v[1] = sbyte<1>(lo); v[2] = sbyte<2>(lo); v[3] = sbyte<3>(lo);
         v[4] = sbyte<0>(hi); v[5] = sbyte<1>(hi); v[6] = sbyte<2>(hi); v[7] = sbyte<3>(hi);
     } else {
-        uint32_t w0, w1;
-        if (kb % 2) {
-            const uint32_t* a = reinterpret_cast<const uint32_t*>(blk + 2 + 8 * g16);
-            w0 = a[0];
-            w1 = a[1];
-        } else {
-            const uint32_t* a = reinterpret_cast<const uint32_t*>(blk + 8 * g16);
-            const uint32_t a0 = a[0], a1 = a[1], a2 = a[2];
-            w0 = __builtin_amdgcn_alignbyte(a1, a0, 2);
-            w1 = __builtin_amdgcn_alignbyte(a2, a1, 2);
+        const uint32_t a0 = a[0], a1 = a[1];
+        uint32_t w0 = a0, w1 = a1;
+        if (ANY || late) {
+            const uint32_t a2 = a[2];
+            w0 = __builtin_amdgcn_alignbyte(a1, a0, late);
+            w1 = __builtin_amdgcn_alignbyte(a2, a1, late);
         }
         v[0] = sbyte<0>(w0); v[1] = sbyte<1>(w0); v[2] = sbyte<2>(w0); v[3] = sbyte<3>(w0);
         v[4] = sbyte<0>(w1); v[5] = sbyte<1>(w1); v[6] = sbyte<2>(w1); v[7] = sbyte<3>(w1);
@@ -72,6 +68,16 @@ __device__ __forceinline__ bf16x8 seg_operand(const uint8_t* unit, int l16, int 
 #pragma unroll
     for (int e = 0; e < 4; ++e) w[e] = bf16_pair(__float_as_uint(v[2 * e]), __float_as_uint(v[2 * e + 1]));
     return __builtin_bit_cast(bf16x8, w);
+}
+
+// The scale of block kb (may differ by lane) of weight row l16.
+template <uint32_t QT, bool ANY>
+__device__ __forceinline__ float seg_scale(const uint8_t* unit, int l16, int kb, int skew) {
+    using U = SegUnit<QT, ANY>;
+    const uint32_t half = *reinterpret_cast<const uint16_t*>(unit + l16 * U::PITCH + kb * U::BB + (ANY ? skew : 0));
+    float d = U::kQ4 ? f16_fast(half) * 0.0625f : f16_fast(half);
+    asm("" : "+v"(d));  // an FP32 value: v_fma_f32 issues at twice v_fma_mix_f32's rate
+    return d;
 }
 
 // A workgroup takes one A tile and 16 N weight rows; its WK waves take the K
@@ -98,9 +104,9 @@ __device__ __forceinline__ bf16x8 seg_operand(const uint8_t* unit, int l16, int 
 // block b + j.  Each block's product is formed with the same operand, a lane
 // keeps the one its output rows belong to, and the row groups are added at
 // the end: the activations of TB blocks are split for the price of one.
-template <uint32_t QT, int NT, int TB, int N, int WK, class Policy>
+template <uint32_t QT, bool ANY, int NT, int TB, int N, int WK, class Policy>
 __global__ __launch_bounds__(WK * kWave) void gemm_thin_kernel(Policy pol, int rows, int cols) {
-    using U = SegUnit<QT>;
+    using U = SegUnit<QT, ANY>;
     static_assert(NT == 1 || TB == 1, "blocks share one A subtile only");
     static_assert(!Policy::kPairedColumns || N % 2 == 0, "paired columns need row tiles in pairs");
     constexpr int TR = 16 / TB;  // A rows of a subtile per block
@@ -125,7 +131,8 @@ __global__ __launch_bounds__(WK * kWave) void gemm_thin_kernel(Policy pol, int r
     const int n0 = (L % pol.tiles_x) * BN;
     const int nblk = cols / kBlock;
     const int row_bytes = nblk * U::BB;
-    const int units = nblk / U::BLOCKS;
+    const int units = (nblk + U::BLOCKS - 1) / U::BLOCKS;
+    const int skew = ANY ? 2 * (l16 & 1 & (row_bytes >> 1)) : 0;  // this lane's weight row starts late by
     uint8_t* const wl = lds + wave * kWaveLds;
     uint8_t* const al = wl + N * U::BYTES;
 
@@ -135,11 +142,13 @@ __global__ __launch_bounds__(WK * kWave) void gemm_thin_kernel(Policy pol, int r
     const float* a_src[kALoads];
 #pragma unroll
     for (int j = 0; j < kALoads; ++j)
-        a_src[j] = pol.a_row(tile, min(j * (8 / CB) + lane / (8 * CB), tile.mcount - 1)) + 4 * (lane % (8 * CB));
+        a_src[j] = pol.a_row(tile, min(j * (8 / CB) + lane / (8 * CB), tile.mcount - 1)) + 4 * (lane % 8);
     f32x4 a_reg[kALoads];
-    auto load_a = [&](int kb) {
+    auto load_a = [&](int kb) {  // blocks past the last read the last
+        const int block = kb + lane % (8 * CB) / 8;
+        const int k = kBlock * (ANY ? min(block, nblk - 1) : block);
 #pragma unroll
-        for (int j = 0; j < kALoads; ++j) a_reg[j] = *reinterpret_cast<const f32x4*>(a_src[j] + kBlock * kb);
+        for (int j = 0; j < kALoads; ++j) a_reg[j] = *reinterpret_cast<const f32x4*>(a_src[j] + k);
     };
     auto store_a = [&]() {
 #pragma unroll
@@ -152,10 +161,13 @@ __global__ __launch_bounds__(WK * kWave) void gemm_thin_kernel(Policy pol, int r
 #pragma unroll
     for (int j = 0; j <= U::WIDE; ++j) {
         const int pos = j < U::WIDE ? 16 * (j * kWave + lane) : U::WIDE * 1024 + 4 * lane;
-        off[j] = pos / U::PITCH * row_bytes + pos % U::PITCH;
+        const int start = pos / U::PITCH * row_bytes;
+        off[j] = (ANY ? start & ~3 : start) + pos % U::PITCH;
     }
     const uint8_t* first[N];  // row 0 of each 16-row unit (uniform)
-    int bytes[N];             // bytes of its valid rows
+    // Bytes of its valid rows, in whole dwords (the buffer range drops a
+    // dword that is not whole; the matrix starts on one).
+    int bytes[N];
 #pragma unroll
     for (int t = 0; t < N; ++t) {
         const int n = n0 + 16 * t;
@@ -163,9 +175,9 @@ __global__ __launch_bounds__(WK * kWave) void gemm_thin_kernel(Policy pol, int r
         const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p));
         const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p >> 32));
         first[t] = reinterpret_cast<const uint8_t*>((static_cast<uintptr_t>(hi) << 32) | lo);
-        bytes[t] = max(0, min(16, rows - n)) * row_bytes;
+        bytes[t] = (max(0, min(16, rows - n)) * row_bytes + 3) & ~3;
     }
-    SegRegs reg[N];
+    SegRegs<U::WIDE> reg[N];
     auto load_units = [&](int u) {  // past the last unit: zeros, no memory touched
         const bool live = u < units;
         const int at = live ? u * U::STEP : 0;
@@ -232,21 +244,15 @@ __global__ __launch_bounds__(WK * kWave) void gemm_thin_kernel(Policy pol, int r
 #pragma unroll
             for (int b = 0; b < G; ++b) {
                 const int kb = c * CB + b * TB;
+                if (ANY && u * U::BLOCKS + kb >= nblk) break;  // a short last unit: whole groups (thin_ok)
 #pragma unroll
                 for (int t = 0; t < N; ++t) {
                     const uint8_t* unit = wl + t * U::BYTES;
                     bf16x8 w[TB];
-                    float d[TB];
 #pragma unroll
-                    for (int j = 0; j < TB; ++j) w[j] = seg_operand<QT>(unit, l16, g16, kb + j, d[j]);
-                    float scale = d[0];
-                    if constexpr (TB > 1) {
-                        // The block this lane's output rows belong to.
-                        const uint32_t half = *reinterpret_cast<const uint16_t*>(unit + l16 * U::PITCH +
-                                                                                 (kb + 4 * g16 / TR) * U::BB);
-                        scale = U::kQ4 ? f16_fast(half) * 0.0625f : f16_fast(half);
-                    }
-                    asm("" : "+v"(scale));  // an FP32 value: v_fma_f32 issues at twice v_fma_mix_f32's rate
+                    for (int j = 0; j < TB; ++j) w[j] = seg_operand<QT, ANY>(unit, l16, g16, kb + j, skew);
+                    // The scale of the block this lane's output rows belong to.
+                    const float scale = seg_scale<QT, ANY>(unit, l16, kb + 4 * g16 / TR, skew);
 #pragma unroll
                     for (int i = 0; i < NT; ++i) {
                         f32x4 sum[TB];
@@ -314,16 +320,15 @@ __global__ __launch_bounds__(WK * kWave) void gemm_thin_kernel(Policy pol, int r
 constexpr int kThinWaves = 8;
 constexpr int kThinMaxRows = 32;  // A rows of the largest tile
 
-// The kernel reads whole units of weight rows 16 bytes at a time: row length
-// a multiple of 256 columns, 16-byte aligned rows and activations.  Against
-// gemm_x3.h's tiles (with a K-split workspace) on Q8_0 and Q4_0 matrices of
-// 128 to 20000 rows and 1024 to 24576 columns it took 0.33-0.58 of the time
-// at 2 and 8 tokens, 0.41-0.73 at 16 and 0.45-0.98 at 32 up to 16384 columns;
-// there, past that length, a wave's K units in turn took 0.65 to 1.08 of
-// it.  From 33 tokens on, gemm_x3.h's 64-row tiles read the weights fewer times.
-inline bool thin_ok(int count, int cols, bool aligned16) {
-    return aligned16 && cols % (8 * kBlock) == 0 && cols <= (1 << 22) && count <= kThinMaxRows &&
-           (count <= 16 || cols <= 16384);
+// Dword-aligned weights (every 16-row unit then starts on a dword, whatever the
+// row length) and 16-byte aligned activations.  Against gemm_x3.h's tiles
+// (with a K-split workspace) on Q8_0 and Q4_0 matrices of 128 to 20000 rows
+// and 1024 to 24576 columns it took 0.33-0.58 of the time at 2 and 8 tokens,
+// 0.41-0.73 at 16 and 0.45-0.98 at 32 up to 16384 columns; there, past that
+// length, a wave's K units in turn took 0.65 to 1.08 of it.  From 33 tokens
+// on, gemm_x3.h's 64-row tiles read the weights fewer times.
+inline bool thin_ok(int count, int cols, bool aligned_ok) {
+    return aligned_ok && cols <= (1 << 22) && count <= kThinMaxRows && (count <= 16 || cols <= 16384);
 }
 
 // Row tiles per workgroup for `rows` weight rows: as many as leave one
@@ -335,16 +340,15 @@ inline int thin_row_tiles(int rows, int count) {
     return per_cu <= 3 ? per_cu : count <= 8 ? 2 : 3;
 }
 
-template <uint32_t QT, int NT, int TB, class P>
-int launch_thin_shape(P pol, int rows, int count, int cols, hipStream_t stream) {
-    constexpr int BM = NT == 1 ? 16 / TB : 16 * NT;
-    const int tiles_y = (count + BM - 1) / BM;
+// `tiles_y` A tiles of the shape's height (for a grouped launch: at most).
+template <uint32_t QT, bool ANY, int NT, int TB, class P>
+int launch_thin_shape(P pol, int rows, int count, int cols, int tiles_y, hipStream_t stream) {
     auto launch = [&](auto n) {
         constexpr int N = decltype(n)::value;
         pol.tiles_x = (rows + 16 * N - 1) / (16 * N);
         const long long tiles = static_cast<long long>(pol.tiles_x) * tiles_y;
         if (tiles > 0x7fffffLL) return static_cast<int>(Q3X_HIP_EINVAL);
-        hipLaunchKernelGGL((gemm_thin_kernel<QT, NT, TB, N, kThinWaves, P>), dim3(static_cast<unsigned>(tiles)),
+        hipLaunchKernelGGL((gemm_thin_kernel<QT, ANY, NT, TB, N, kThinWaves, P>), dim3(static_cast<unsigned>(tiles)),
                            dim3(kThinWaves * kWave), 0, stream, pol, rows, cols);
         return launch_status();
     };
@@ -362,12 +366,23 @@ int launch_thin_shape(P pol, int rows, int count, int cols, hipStream_t stream) 
 // One launch over `count` A rows and `rows` weight rows (thin_ok).  7 x 12288
 // x 4096 Q8_0 16 us (43 on gemm_x3.h's tiles; a matvec of it 12), 24 rows 24
 // (45); 7 x 17408 x 5120 Q4_0 25 us (63); 7 x 1024 x 4096 8 us (16).  The A tile is the smallest that holds the rows.
+template <uint32_t QT, bool ANY, class P>
+int launch_thin_rows(const P& pol, int rows, int count, int cols, hipStream_t stream) {
+    // A group of TB blocks must not straddle the row's end.
+    const int nblk = cols / kBlock;
+    if (count <= 4 && (!ANY || nblk % 4 == 0)) return launch_thin_shape<QT, ANY, 1, 4>(pol, rows, count, cols, 1, stream);
+    if (count <= 8 && (!ANY || nblk % 2 == 0)) return launch_thin_shape<QT, ANY, 1, 2>(pol, rows, count, cols, 1, stream);
+    if (count <= 16) return launch_thin_shape<QT, ANY, 1, 1>(pol, rows, count, cols, 1, stream);
+    return launch_thin_shape<QT, ANY, 2, 1>(pol, rows, count, cols, 1, stream);
+}
+
+// Rows of whole units, 16-byte aligned?
+inline bool thin_whole(int cols, bool aligned16) { return aligned16 && cols % (8 * kBlock) == 0; }
+
 template <uint32_t QT, class P>
-int launch_thin(const P& pol, int rows, int count, int cols, hipStream_t stream) {
-    if (count <= 4) return launch_thin_shape<QT, 1, 4>(pol, rows, count, cols, stream);
-    if (count <= 8) return launch_thin_shape<QT, 1, 2>(pol, rows, count, cols, stream);
-    if (count <= 16) return launch_thin_shape<QT, 1, 1>(pol, rows, count, cols, stream);
-    return launch_thin_shape<QT, 2, 1>(pol, rows, count, cols, stream);
+int launch_thin(const P& pol, int rows, int count, int cols, bool aligned16, hipStream_t stream) {
+    return thin_whole(cols, aligned16) ? launch_thin_rows<QT, false>(pol, rows, count, cols, stream)
+                                       : launch_thin_rows<QT, true>(pol, rows, count, cols, stream);
 }
 
 }  // namespace q3x

@@ -1449,9 +1449,10 @@ int q3x::gate_up_swiglu(const void* gate, const void* up, uint32_t type, int I, 
     g.X = X; g.cols = H; g.count = count;
     g.gate = static_cast<const uint8_t*>(gate); g.up = static_cast<const uint8_t*>(up);
     g.row_bytes = static_cast<size_t>(H / kBlock) * block_bytes(type); g.I = I; g.h = h;
-    if (thin_ok(count, H, aligned(gate, 16) && aligned(up, 16)))
-        return type == Q3X_HIP_MATRIX_Q8_0 ? launch_thin<Q3X_HIP_MATRIX_Q8_0>(g, 2 * I, count, H, stream)
-                                           : launch_thin<Q3X_HIP_MATRIX_Q4_0>(g, 2 * I, count, H, stream);
+    const bool aligned16 = aligned(gate, 16) && aligned(up, 16);
+    if (thin_ok(count, H, aligned(gate, 4) && aligned(up, 4)))
+        return type == Q3X_HIP_MATRIX_Q8_0 ? launch_thin<Q3X_HIP_MATRIX_Q8_0>(g, 2 * I, count, H, aligned16, stream)
+                                           : launch_thin<Q3X_HIP_MATRIX_Q4_0>(g, 2 * I, count, H, aligned16, stream);
     return type == Q3X_HIP_MATRIX_Q8_0 ? launch_token_gemm<Q3X_HIP_MATRIX_Q8_0>(g, 2 * I, stream)
                                        : launch_token_gemm<Q3X_HIP_MATRIX_Q4_0>(g, 2 * I, stream);
 }

@@ -29,7 +29,8 @@ def _run(type_, w, rows, cols, X, offset, add):
 @pytest.mark.parametrize("type_", [Q8_0, Q4_0])
 @pytest.mark.parametrize("tokens", [1, 4, 5, 8, 9, 16, 17, 32, 33])
 @pytest.mark.parametrize("rows,cols", [(1, 256), (15, 512), (49, 2304), (33, 4096), (4097, 1024), (8200, 256),
-                                       (12300, 256)])
+                                       (12300, 256), (1, 32), (33, 32), (17, 96), (31, 160), (100, 288), (3, 1056),
+                                       (47, 4128), (18, 4160), (8200, 96)])
 def test_few_token_gemm(type_, tokens, rows, cols):
     rng = np.random.default_rng(type_ + tokens * 64 + rows)
     w = random_blocks(rng, type_, rows, cols)
@@ -43,6 +44,8 @@ def test_few_token_gemm(type_, tokens, rows, cols):
     # Reading 3 back after adding costs up to half an ulp of the sum.
     added = _run(type_, w, rows, cols, X, 0, True)
     assert np.all(np.abs(added - want) <= bound + 2.0 ** -23 * (3.0 + np.abs(want)))
+    dword = _run(type_, w, rows, cols, X, 4, False)  # a matrix aligned to 4 bytes only
+    assert np.all(np.abs(dword - want) <= bound)
     general = _run(type_, w, rows, cols, X, 2, False)
     # Two FP32 sums of the same exact products: at most 2 (K + 40) 2^-24 of
     # the sum of their magnitudes, far below the bound above.
