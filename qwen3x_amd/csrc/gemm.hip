@@ -75,7 +75,7 @@ int gemm(const void* w, uint32_t type, int rows, int cols, const float* X, int c
     }
     // A few tokens: the launch that reads the weights once, in whole row
     // segments (launch_thin).
-    if (thin_ok(count, cols, aligned(w, 4))) {
+    if (thin_ok(count, rows, cols, aligned(w, 4))) {
         DenseGemm t{0, X, cols, count, static_cast<const uint8_t*>(w), row_bytes, Y, rows, accumulate != 0};
         return type == Q3X_HIP_MATRIX_Q8_0 ? launch_thin<Q3X_HIP_MATRIX_Q8_0>(t, rows, count, cols, aligned(w, 16), stream)
                                            : launch_thin<Q3X_HIP_MATRIX_Q4_0>(t, rows, count, cols, aligned(w, 16), stream);

@@ -327,8 +327,8 @@ constexpr int kThinMaxRows = 32;  // A rows of the largest tile
 // 0.41-0.73 at 16 and 0.45-0.98 at 32 up to 16384 columns; there, past that
 // length, a wave's K units in turn took 0.65 to 1.08 of it.  From 33 tokens
 // on, gemm_x3.h's 64-row tiles read the weights fewer times.
-inline bool thin_ok(int count, int cols, bool aligned_ok) {
-    return aligned_ok && cols <= (1 << 22) && count <= kThinMaxRows && (count <= 16 || cols <= 16384);
+inline bool thin_ok(int count, int rows, int cols, bool aligned_ok) {
+    return aligned_ok && cols <= (1 << 22) && rows <= (1 << 26) && count <= kThinMaxRows && (count <= 16 || cols <= 16384);
 }
 
 // Row tiles per workgroup for `rows` weight rows: as many as leave one
@@ -341,18 +341,18 @@ inline int thin_row_tiles(int rows, int count) {
 }
 
 // `tiles_y` A tiles of the shape's height (for a grouped launch: at most).
-template <uint32_t QT, bool ANY, int NT, int TB, class P>
+template <uint32_t QT, bool ANY, int NT, int TB, int WK, class P>
 int launch_thin_shape(P pol, int rows, int count, int cols, int tiles_y, hipStream_t stream) {
     auto launch = [&](auto n) {
         constexpr int N = decltype(n)::value;
         pol.tiles_x = (rows + 16 * N - 1) / (16 * N);
         const long long tiles = static_cast<long long>(pol.tiles_x) * tiles_y;
         if (tiles > 0x7fffffLL) return static_cast<int>(Q3X_HIP_EINVAL);
-        hipLaunchKernelGGL((gemm_thin_kernel<QT, ANY, NT, TB, N, kThinWaves, P>), dim3(static_cast<unsigned>(tiles)),
-                           dim3(kThinWaves * kWave), 0, stream, pol, rows, cols);
+        hipLaunchKernelGGL((gemm_thin_kernel<QT, ANY, NT, TB, N, WK, P>), dim3(static_cast<unsigned>(tiles)),
+                           dim3(WK * kWave), 0, stream, pol, rows, cols);
         return launch_status();
     };
-    if constexpr (P::kPairedColumns) {
+    if constexpr (P::kPairedColumns || P::kPartialTiles) {
         return launch(std::integral_constant<int, 2>{});
     } else {
         switch (thin_row_tiles(rows, count)) {
@@ -370,10 +370,10 @@ template <uint32_t QT, bool ANY, class P>
 int launch_thin_rows(const P& pol, int rows, int count, int cols, hipStream_t stream) {
     // A group of TB blocks must not straddle the row's end.
     const int nblk = cols / kBlock;
-    if (count <= 4 && (!ANY || nblk % 4 == 0)) return launch_thin_shape<QT, ANY, 1, 4>(pol, rows, count, cols, 1, stream);
-    if (count <= 8 && (!ANY || nblk % 2 == 0)) return launch_thin_shape<QT, ANY, 1, 2>(pol, rows, count, cols, 1, stream);
-    if (count <= 16) return launch_thin_shape<QT, ANY, 1, 1>(pol, rows, count, cols, 1, stream);
-    return launch_thin_shape<QT, ANY, 2, 1>(pol, rows, count, cols, 1, stream);
+    if (count <= 4 && (!ANY || nblk % 4 == 0)) return launch_thin_shape<QT, ANY, 1, 4, kThinWaves>(pol, rows, count, cols, 1, stream);
+    if (count <= 8 && (!ANY || nblk % 2 == 0)) return launch_thin_shape<QT, ANY, 1, 2, kThinWaves>(pol, rows, count, cols, 1, stream);
+    if (count <= 16) return launch_thin_shape<QT, ANY, 1, 1, kThinWaves>(pol, rows, count, cols, 1, stream);
+    return launch_thin_shape<QT, ANY, 2, 1, kThinWaves>(pol, rows, count, cols, 1, stream);
 }
 
 // Rows of whole units, 16-byte aligned?
@@ -383,6 +383,34 @@ template <uint32_t QT, class P>
 int launch_thin(const P& pol, int rows, int count, int cols, bool aligned16, hipStream_t stream) {
     return thin_whole(cols, aligned16) ? launch_thin_rows<QT, false>(pol, rows, count, cols, stream)
                                        : launch_thin_rows<QT, true>(pol, rows, count, cols, stream);
+}
+
+// A grouped launch (a tile table on the device, at most `tiles_y` tiles of
+// `height` rows, about `tiles` of them live): two row tiles a workgroup.  K is
+// split over as many waves as the chip holds at once (16 a CU), no more: a wave
+// waits some microseconds for its first unit whatever follows.
+template <uint32_t QT, bool ANY, class P>
+int launch_thin_grouped(const P& pol, int height, int rows, int cols, int tiles_y, double tiles, hipStream_t stream) {
+    using U = SegUnit<QT, ANY>;
+    const int units = (cols / kBlock + U::BLOCKS - 1) / U::BLOCKS;
+    const double split = std::min<double>(units, 16.0 * kCUs / (tiles * ((rows + 31) / 32)));
+    auto waves = [&](auto nt, auto tb) {
+        constexpr int NT = decltype(nt)::value, TB = decltype(tb)::value;
+        if (split >= 6.0) return launch_thin_shape<QT, ANY, NT, TB, 8>(pol, rows, height, cols, tiles_y, stream);
+        if (split >= 3.0) return launch_thin_shape<QT, ANY, NT, TB, 4>(pol, rows, height, cols, tiles_y, stream);
+        if (split >= 1.5) return launch_thin_shape<QT, ANY, NT, TB, 2>(pol, rows, height, cols, tiles_y, stream);
+        return launch_thin_shape<QT, ANY, NT, TB, 1>(pol, rows, height, cols, tiles_y, stream);
+    };
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I4 = std::integral_constant<int, 4>;
+    // Blocks share operand registers only where they do not straddle the row's
+    // end; a taller tile shape takes a shorter tile too.
+    const int nblk = cols / kBlock;
+    if (height <= 4 && (!ANY || nblk % 4 == 0)) return waves(I1{}, I4{});
+    if (height <= 8 && (!ANY || nblk % 2 == 0)) return waves(I1{}, I2{});
+    if (height <= 16) return waves(I1{}, I1{});
+    return waves(I2{}, I1{});
 }
 
 }  // namespace q3x

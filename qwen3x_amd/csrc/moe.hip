@@ -23,6 +23,8 @@
 // No atomics touch any accumulated value, so results are deterministic.
 #include "moe.h"
 
+#include <cmath>
+
 #include "gemm.h"
 #include "gemm_thin.h"
 #include "gemm_x3.h"
@@ -307,17 +309,38 @@ struct MoeLayout {
     int chunks;
     size_t gu, h, d, total;
     int max_tiles;
+    int thin;  // tile height of the few-pair grouped GEMMs; 0: the 80-pair tiles
 };
 
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
-inline MoeLayout moe_layout(int tokens, int experts, int top_k, int H, int I) {
+// Tile height of the few-pair grouped GEMMs (gemm_thin.h) for a launch whose
+// selected experts get `mean` pairs on average, 0 where the 80-pair tiles
+// are faster: the height that holds the mean and a standard deviation or so,
+// since an expert past it takes a second tile and reads its weights (from the
+// caches) again.  Measured, whole layers, few-pair / 80-pair us: 256 experts
+// top 8, H 2048, I 512, Q4_0: 5 tokens 61 / 96, 19 104 / 159, 64 170 / 277,
+// 180 254 / 314, 300 (11 pairs an expert) 271 / 343; Q8_0 19 148 / 204, 300
+// 362 / 436.  32-row tiles only where few experts leave the 80-pair launch
+// short of workgroups: 8 experts top 8, H 3072, I 1024, Q8_0, 19 tokens 90 /
+// 151, but 32 experts top 2 at 200 tokens 128 / 111.
+inline double moe_live_experts(int tokens, int experts, int top_k) {
+    return experts * (1.0 - std::pow(1.0 - static_cast<double>(std::min(top_k, experts)) / experts, tokens));
+}
+inline int moe_thin_height(int tokens, int experts, int top_k) {
+    const double live = moe_live_experts(tokens, experts, top_k);
+    const double mean = static_cast<double>(tokens) * top_k / live;
+    return mean <= 2.0 ? 4 : mean <= 5.0 ? 8 : mean <= 11.0 ? 16 : mean <= 24.0 && live <= 16.0 ? 32 : 0;
+}
+
+inline MoeLayout moe_layout(int tokens, int experts, int top_k, int H, int I, int thin) {
     MoeLayout L{};
     const size_t P = static_cast<size_t>(tokens) * top_k;
     size_t off = 0;
     auto take = [&](size_t bytes) { const size_t at = off; off = align_up(off + bytes, 256); return at; };
     {  // grouping arrays (also for one token: the fallback of unaligned decode shapes)
-        L.max_tiles = static_cast<int>(P / kGrpBM + std::min<size_t>(experts, P) + 1);
+        L.thin = thin;
+        L.max_tiles = static_cast<int>(P / (thin ? thin : kGrpBM) + std::min<size_t>(experts, P) + 1);
         L.ntiles = take(sizeof(int));
         L.nvalid = take(sizeof(int));
         L.tile_expert = take(sizeof(int) * L.max_tiles);
@@ -332,6 +355,19 @@ inline MoeLayout moe_layout(int tokens, int experts, int top_k, int H, int I) {
     L.h = take(sizeof(float) * P * I);
     L.d = take(sizeof(float) * P * H);
     L.total = off;
+    return L;
+}
+
+inline MoeLayout moe_layout(int tokens, int experts, int top_k, int H, int I) {
+    const MoeLayout wide = moe_layout(tokens, experts, top_k, H, I, 0);
+    const int thin = tokens > 1 ? moe_thin_height(tokens, experts, top_k) : 0;
+    if (thin == 0) return wide;
+    const MoeLayout L = moe_layout(tokens, experts, top_k, H, I, thin);
+    // More tiles than a grid holds stay on the wide ones.
+    if (static_cast<long long>(L.max_tiles) * (std::max(2LL * I, static_cast<long long>(H)) / 32 + 1) > (1 << 22)) return wide;
+    // The longer tile table must not push a request past the static scratch
+    // that held it.
+    if (L.total > Q3X_HIP_NOALLOC_SCRATCH_BYTES && wide.total <= Q3X_HIP_NOALLOC_SCRATCH_BYTES) return wide;
     return L;
 }
 
@@ -869,13 +905,42 @@ struct GroupedShared {
     const uint8_t* down = nullptr;
 };
 
-template <uint32_t QT, int WM, int WN, int SM, int SN>
-int moe_grouped_tiles(const uint8_t* gate_up, const uint8_t* down, int experts, int H, int I, const float* X,
+// The grouped GEMM of policy g over `rows` weight rows of K = cols, at most
+// `tiles_bound` tiles: few-pair tiles of height `thin`, or 80 x 256 on 8 waves
+// of 80x32.
+//
+// 80 pairs x 256 weight rows: at 2048 tokens x top
+// 8 of 256 experts an expert averages 64 pairs (standard deviation about
+// 8): 64-pair tiles give about half of the experts a second, nearly
+// empty tile that brings the expert's weight rows into the CU again (378
+// tiles for 256 experts at config 4), 80-pair tiles give 261, and the
+// 80x32 wave tile keeps the register count at 128, so two workgroups
+// still share a CU.  Alternating runs of one box at config 4: 197-201
+// TFLOP/s against 188-192 for 64 x 256 on 8 waves of 32x64; 96 x 256 on
+// 12 waves of 32x64 (one workgroup a CU) 191-193, on 8 waves of 48x64
+// (164 registers) 182.  Earlier, with 64-pair tiles: 64 x 128 on 32x32
+// waves, 64 x 512 on 8 waves of 64x64 or 32x128, 64 x 256 on 8 waves of
+// 64x32, on 4 of 64x64 or on 16 of 32x32, and 64 x 128 on 4 waves of
+// 32x64 all ran slower than 64 x 256 on 32x64 waves.
+constexpr int kWideBM = 80, kWideBN = 256;
+
+template <uint32_t QT, class P>
+int launch_grouped(P g, int thin, bool aligned16, int rows, int cols, int tiles_bound, double tiles, hipStream_t stream) {
+    if (thin)
+        return thin_whole(cols, aligned16) ? launch_thin_grouped<QT, false>(g, thin, rows, cols, tiles_bound, tiles, stream)
+                                           : launch_thin_grouped<QT, true>(g, thin, rows, cols, tiles_bound, tiles, stream);
+    static_assert(kWideBM >= kGrpBM, "the workspace bounds the tile count for kGrpBM-pair tiles");
+    g.tiles_x = (rows + kWideBN - 1) / kWideBN;
+    hipLaunchKernelGGL((gemm_x3_kernel<QT, 1, 8, 5, 2, P, 1, kGrpCF>), dim3(g.tiles_x * tiles_bound), dim3(8 * kWave), 0,
+                       stream, g, rows, cols);
+    return launch_status();
+}
+
+template <uint32_t QT>
+int moe_grouped(const uint8_t* gate_up, const uint8_t* down, int experts, int H, int I, const float* X,
                 int tokens, const int* ids, const float* weights, int top_k, float* Y, int accumulate,
-                uint8_t* ws, const MoeLayout& L, hipStream_t stream, const GroupedShared& shared) {
+                uint8_t* ws, const MoeLayout& L, hipStream_t stream, const GroupedShared& shared = {}) {
     constexpr int BB = QT == Q3X_HIP_MATRIX_Q8_0 ? kQ8Bytes : kQ4Bytes;
-    constexpr int BM = WM * SM * 16, BN = WN * SN * 16, NT = WM * WN * kWave;
-    static_assert(BM >= kGrpBM, "the workspace bounds the tile count for kGrpBM-pair tiles");
     const int P = tokens * top_k;
     int* ntiles = reinterpret_cast<int*>(ws + L.ntiles);
     int* nvalid = reinterpret_cast<int*>(ws + L.nvalid);
@@ -888,55 +953,58 @@ int moe_grouped_tiles(const uint8_t* gate_up, const uint8_t* down, int experts, 
     float* h = reinterpret_cast<float*>(ws + L.h);
     float* d = reinterpret_cast<float*>(ws + L.d);
 
+    // Few-pair tiles need every expert matrix to start on a dword.
+    const size_t gu_row = static_cast<size_t>(H / kBlock) * BB;
+    const size_t down_row = static_cast<size_t>(I / kBlock) * BB;
+    auto shared_aligned = [&](size_t a) {
+        return shared.group < 0 || (aligned(shared.gate, a) && aligned(shared.up, a) && aligned(shared.down, a));
+    };
+    const bool dwords = aligned(gate_up, 4) && aligned(down, 4) && shared_aligned(4) && gu_row * I % 4 == 0 &&
+                        down_row * H % 4 == 0;
+    const int thin = dwords ? L.thin : 0;
+    const bool aligned16 = aligned(gate_up, 16) && aligned(down, 16) && shared_aligned(16);
+
     int* chunk_counts = reinterpret_cast<int*>(ws + L.chunk_counts);
     hipLaunchKernelGGL(moe_rank_kernel, dim3(L.chunks), dim3(kChunk), 0, stream, ids, P, experts, chunk_counts,
                        pos_of_pair);
     int status = launch_status();
     if (status != Q3X_HIP_OK) return status;
     hipLaunchKernelGGL(moe_place_kernel, dim3(L.chunks), dim3(kGroupThreads), 0, stream,
-                       static_cast<const int*>(chunk_counts), L.chunks, experts, BM, tile_expert, tile_start,
+                       static_cast<const int*>(chunk_counts), L.chunks, experts, thin ? thin : kWideBM, tile_expert, tile_start,
                        tile_count, ntiles, nvalid, ids, P, top_k, pos_of_pair, src_token);
     if ((status = launch_status()) != Q3X_HIP_OK) return status;
 
-    const size_t gu_row = static_cast<size_t>(H / kBlock) * BB;
-    const size_t down_row = static_cast<size_t>(I / kBlock) * BB;
     const int tiles_bound = L.max_tiles;
+    const double tiles = moe_live_experts(tokens, experts, top_k);  // live tiles, about
     if (I % 64 == 0) {
         // SwiGLU in the gate_up epilogue: h directly.
         GroupedGateUp g1{};
-        const int nx = (2 * I + BN - 1) / BN;
-        static_cast<GroupedGemm&>(g1) = GroupedGemm{nx, X, H, src_token, gate_up, gu_row * 2 * I, gu_row,
+        static_cast<GroupedGemm&>(g1) = GroupedGemm{0, X, H, src_token, gate_up, gu_row * 2 * I, gu_row,
                                                     tile_expert, tile_start, tile_count, ntiles, nullptr, 0};
         g1.I = I;
         g1.h = h;
         g1.shared_group = shared.group;
         g1.shared_rows = shared.gate;
         g1.shared_up = shared.up;
-        hipLaunchKernelGGL((gemm_x3_kernel<QT, WM, WN, SM, SN, GroupedGateUp, 1, kGrpCF>), dim3(nx * tiles_bound), dim3(NT), 0,
-                           stream, g1, 2 * I, H);
-        if ((status = launch_status()) != Q3X_HIP_OK) return status;
+        if ((status = launch_grouped<QT>(g1, thin, aligned16, 2 * I, H, tiles_bound, tiles, stream)) != Q3X_HIP_OK)
+            return status;
     } else {
         if (shared.group >= 0) return Q3X_HIP_ENOTSUP;  // a shared group needs the paired gate_up
-        const int nx = (2 * I + BN - 1) / BN;
-        GroupedGemm g1{nx, X, H, src_token, gate_up, gu_row * 2 * I, gu_row, tile_expert, tile_start, tile_count,
+        GroupedGemm g1{0, X, H, src_token, gate_up, gu_row * 2 * I, gu_row, tile_expert, tile_start, tile_count,
                        ntiles, gu, 2 * I};
-        hipLaunchKernelGGL((gemm_x3_kernel<QT, WM, WN, SM, SN, GroupedGemm, 1, kGrpCF>), dim3(nx * tiles_bound), dim3(NT), 0,
-                           stream, g1, 2 * I, H);
-        if ((status = launch_status()) != Q3X_HIP_OK) return status;
+        if ((status = launch_grouped<QT>(g1, thin, aligned16, 2 * I, H, tiles_bound, tiles, stream)) != Q3X_HIP_OK)
+            return status;
         const size_t sw = static_cast<size_t>(P) * I;
         const int sw_blocks = static_cast<int>(std::min<size_t>((sw + 255) / 256, 65536));
         hipLaunchKernelGGL(swiglu_kernel, dim3(sw_blocks), dim3(256), 0, stream, gu, h, I, 0,
                            static_cast<const int*>(nvalid));
         if ((status = launch_status()) != Q3X_HIP_OK) return status;
     }
-    const int nx2 = (H + BN - 1) / BN;
-    GroupedGemm g2{nx2, h, I, nullptr, down, down_row * H, down_row, tile_expert, tile_start, tile_count,
+    GroupedGemm g2{0, h, I, nullptr, down, down_row * H, down_row, tile_expert, tile_start, tile_count,
                    ntiles, d, H};
     g2.shared_group = shared.group;
     g2.shared_rows = shared.down;
-    hipLaunchKernelGGL((gemm_x3_kernel<QT, WM, WN, SM, SN, GroupedGemm, 1, kGrpCF>), dim3(nx2 * tiles_bound), dim3(NT), 0,
-                       stream, g2, H, I);
-    if ((status = launch_status()) != Q3X_HIP_OK) return status;
+    if ((status = launch_grouped<QT>(g2, thin, aligned16, H, I, tiles_bound, tiles, stream)) != Q3X_HIP_OK) return status;
     const size_t outs = static_cast<size_t>(tokens) * H;
     if (H % 4 == 0 && aligned(Y, 16)) {
         hipLaunchKernelGGL(combine4_kernel, dim3(static_cast<unsigned>((outs / 4 + 255) / 256)), dim3(256), 0,
@@ -946,27 +1014,6 @@ int moe_grouped_tiles(const uint8_t* gate_up, const uint8_t* down, int experts, 
     hipLaunchKernelGGL(combine_kernel, dim3(static_cast<unsigned>((outs + 255) / 256)), dim3(256), 0,
                        stream, d, pos_of_pair, ids, experts, weights, tokens, top_k, H, Y, accumulate);
     return launch_status();
-}
-
-template <uint32_t QT>
-int moe_grouped(const uint8_t* gate_up, const uint8_t* down, int experts, int H, int I, const float* X,
-                int tokens, const int* ids, const float* weights, int top_k, float* Y, int accumulate,
-                uint8_t* ws, const MoeLayout& L, hipStream_t stream, const GroupedShared& shared = {}) {
-    // 80 pairs x 256 weight rows on 8 waves of 80x32.  At 2048 tokens x top
-    // 8 of 256 experts an expert averages 64 pairs (standard deviation about
-    // 8): 64-pair tiles give about half of the experts a second, nearly
-    // empty tile that brings the expert's weight rows into the CU again (378
-    // tiles for 256 experts at config 4), 80-pair tiles give 261, and the
-    // 80x32 wave tile keeps the register count at 128, so two workgroups
-    // still share a CU.  Alternating runs of one box at config 4: 197-201
-    // TFLOP/s against 188-192 for 64 x 256 on 8 waves of 32x64; 96 x 256 on
-    // 12 waves of 32x64 (one workgroup a CU) 191-193, on 8 waves of 48x64
-    // (164 registers) 182.  Earlier, with 64-pair tiles: 64 x 128 on 32x32
-    // waves, 64 x 512 on 8 waves of 64x64 or 32x128, 64 x 256 on 8 waves of
-    // 64x32, on 4 of 64x64 or on 16 of 32x32, and 64 x 128 on 4 waves of
-    // 32x64 all ran slower than 64 x 256 on 32x64 waves.
-    return moe_grouped_tiles<QT, 1, 8, 5, 2>(gate_up, down, experts, H, I, X, tokens, ids, weights, top_k, Y,
-                                             accumulate, ws, L, stream, shared);
 }
 
 // ------------------------------------------------------------ MoE layer ----
@@ -1450,7 +1497,7 @@ int q3x::gate_up_swiglu(const void* gate, const void* up, uint32_t type, int I, 
     g.gate = static_cast<const uint8_t*>(gate); g.up = static_cast<const uint8_t*>(up);
     g.row_bytes = static_cast<size_t>(H / kBlock) * block_bytes(type); g.I = I; g.h = h;
     const bool aligned16 = aligned(gate, 16) && aligned(up, 16);
-    if (thin_ok(count, H, aligned(gate, 4) && aligned(up, 4)))
+    if (thin_ok(count, 2 * I, H, aligned(gate, 4) && aligned(up, 4)))
         return type == Q3X_HIP_MATRIX_Q8_0 ? launch_thin<Q3X_HIP_MATRIX_Q8_0>(g, 2 * I, count, H, aligned16, stream)
                                            : launch_thin<Q3X_HIP_MATRIX_Q4_0>(g, 2 * I, count, H, aligned16, stream);
     return type == Q3X_HIP_MATRIX_Q8_0 ? launch_token_gemm<Q3X_HIP_MATRIX_Q8_0>(g, 2 * I, stream)

@@ -7,9 +7,10 @@ aligned) within the two paths' FP32 rounding."""
 import numpy as np
 import pytest
 
+import oracle
 import qwen3x_amd as q3x
 from tests.helpers import Q4_0, Q8_0, dequant_numpy, random_blocks, row_bound
-from tests.test_gpu_parity import _torch, dev, host, say
+from tests.test_gpu_parity import _torch, dev, host, moe_bound, say
 
 pytestmark = pytest.mark.gpu
 
@@ -70,3 +71,47 @@ def test_few_token_gemm_keeps_tokens_apart(type_, tokens):
         keep = [t for t in range(tokens) if t != 1]
         assert np.array_equal(got[keep], clean[keep])
         assert not np.isfinite(got[1]).all()
+
+
+@pytest.mark.parametrize("type_", [Q8_0, Q4_0])
+@pytest.mark.parametrize("E,k,tokens", [(16, 2, 2), (16, 2, 4), (8, 2, 12), (4, 2, 20), (4, 2, 40), (300, 1, 5)])
+@pytest.mark.parametrize("H,I", [(256, 256), (288, 96), (320, 160), (1056, 32)])
+def test_few_pair_experts(type_, E, k, tokens, H, I):
+    """The routed experts where an expert gets few pairs: every tile height
+    (4, 8, 16, 32 pairs), spread and skewed routing (one expert holding every
+    token: many tiles of it), ids out of range, rows of any block count.
+    Against the oracle, and against the 80-pair tiles (reached through pools
+    that are not dword aligned)."""
+    torch = _torch()
+    rng = np.random.default_rng(E * 100 + tokens + H)
+    gu = random_blocks(rng, type_, E * 2 * I, H).reshape(-1)
+    dn = random_blocks(rng, type_, E * H, I).reshape(-1)
+    X = rng.normal(0, 1, (tokens, H)).astype(np.float32)
+    wts = rng.uniform(0.1, 1, (tokens, k)).astype(np.float32)
+    for routing in ("spread", "skewed"):
+        ids = np.stack([rng.permutation(E)[:k] for _ in range(tokens)]).astype(np.int32)
+        if routing == "skewed":
+            ids[:, 0] = E - 1
+            ids[ids[:, 1 % k] == E - 1, 1 % k] = 0 if k > 1 else E - 1
+            ids[0, 0] = E  # out of range: contributes nothing
+        say(f"few-pair experts type={type_} E={E} k={k} T={tokens} H={H} I={I} {routing}")
+        valid = ids < E
+        want = oracle.moe_routed(gu, dn, type_, E, H, I, X, np.where(valid, ids, 0).astype(np.int32),
+                                 np.where(valid, wts, 0).astype(np.float32))
+        bound = moe_bound(gu, dn, type_, E, H, I, X, ids, wts)
+        got = []
+        for offset in (0, 2):
+            pools = []
+            for w in (gu, dn):
+                buf = torch.zeros(offset + w.size, dtype=torch.uint8, device="cuda:0")
+                buf[offset:] = dev(w)
+                pools.append(buf[offset:])
+            Y = torch.full((tokens * H + 4,), 5.0, dtype=torch.float32, device="cuda:0")
+            q3x.moe_routed(q3x.ExpertLinear(pools[0], E, 2 * I, H, type_), q3x.ExpertLinear(pools[1], E, H, I, type_),
+                           dev(X), tokens, dev(ids), dev(wts), k, Y)
+            y = host(Y)
+            assert np.all(y[tokens * H:] == 5.0)
+            got.append(y[:tokens * H].reshape(tokens, H))
+        assert np.all(np.abs(got[0] - want) <= bound)
+        # The two tile shapes: the same exact products in FP32 sums of another order.
+        assert np.all(np.abs(got[0].astype(np.float64) - got[1]) <= 2 * bound)
