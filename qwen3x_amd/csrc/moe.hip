@@ -393,6 +393,42 @@ __device__ int block_exclusive_scan(int v, int* buf) {
     return before + x - v;
 }
 
+// The lane's rank among the wave's lanes with the same expert (one ballot per
+// distinct id); the first of them leaves their count in counts[e].
+__device__ int wave_rank(int e, int experts, int* counts) {
+    const int lane = threadIdx.x & (kWave - 1);
+    uint64_t same = 0;
+    uint64_t open = __ballot(1);
+    while (open) {
+        const int v = __builtin_amdgcn_readlane(e, __builtin_ctzll(open));
+        const uint64_t m = __ballot(e == v);
+        if (e == v) same = m;
+        open &= ~m;
+    }
+    const int rank = __popcll(same & ((1ull << lane) - 1));
+    if (e >= 0 && e < experts && rank == 0) counts[e] = __popcll(same);
+    return rank;
+}
+
+// The tile table of a workgroup whose thread e holds expert e's pair count
+// (0 past the experts) and group start.
+__device__ void write_tiles(int total, int start, int bm, int* buf, int* __restrict__ tile_expert,
+                            int* __restrict__ tile_start, int* __restrict__ tile_count, int* __restrict__ ntiles,
+                            int* __restrict__ nvalid) {
+    const int e = threadIdx.x;
+    const int tiles = (total + bm - 1) / bm;
+    const int tile0 = block_exclusive_scan(tiles, buf);
+    for (int j = 0; j < tiles; ++j) {
+        tile_expert[tile0 + j] = e;
+        tile_start[tile0 + j] = start + j * bm;
+        tile_count[tile0 + j] = min(bm, total - j * bm);
+    }
+    if (e == kGroupThreads - 1) {
+        *ntiles = tile0 + tiles;
+        *nvalid = start + total;
+    }
+}
+
 // Stable counting sort of the (token, slot) pairs by expert, in two
 // launches: per chunk of kChunk pairs, the expert histogram and each pair's
 // rank -- the number of earlier pairs of its chunk with the same expert:
@@ -411,22 +447,11 @@ __global__ __launch_bounds__(kChunk) void moe_rank_kernel(const int* __restrict_
     __shared__ int wave_count[kWaves][kRouterMaxExperts];  // per wave and expert: count, then exclusive base
     for (int i = threadIdx.x; i < kWaves * experts; i += kChunk) wave_count[i / experts][i % experts] = 0;
     __syncthreads();
-    const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
     const int p = blockIdx.x * kChunk + threadIdx.x;
     const int e = p < P ? ids[p] : -1;
     const bool valid = e >= 0 && e < experts;
-    // Lanes of this wave with the same id: one ballot per distinct id.
-    uint64_t same = 0;
-    uint64_t open = __ballot(1);
-    while (open) {
-        const int v = __builtin_amdgcn_readlane(e, __builtin_ctzll(open));
-        const uint64_t m = __ballot(e == v);
-        if (e == v) same = m;
-        open &= ~m;
-    }
-    const int rank_in_wave = __popcll(same & ((1ull << lane) - 1));
-    if (valid && rank_in_wave == 0) wave_count[wave][e] = __popcll(same);
+    const int rank_in_wave = wave_rank(e, experts, wave_count[wave]);
     __syncthreads();
     for (int x = threadIdx.x; x < experts; x += kChunk) {
         int run = 0;
@@ -463,16 +488,7 @@ __global__ __launch_bounds__(kGroupThreads) void moe_place_kernel(
     }
     const int start = block_exclusive_scan(total, buf);
     if (owner) chunk_base[e] = start + before;
-    if (blockIdx.x == 0) {
-        const int tiles = owner ? (total + bm - 1) / bm : 0;
-        const int tile0 = block_exclusive_scan(tiles, buf);
-        for (int j = 0; j < tiles; ++j) {
-            tile_expert[tile0 + j] = e;
-            tile_start[tile0 + j] = start + j * bm;
-            tile_count[tile0 + j] = min(bm, total - j * bm);
-        }
-        if (e == kGroupThreads - 1) { *ntiles = tile0 + tiles; *nvalid = start + total; }
-    }
+    if (blockIdx.x == 0) write_tiles(total, start, bm, buf, tile_expert, tile_start, tile_count, ntiles, nvalid);
     __syncthreads();
     // This chunk's pairs at base + rank (moe_rank_kernel's rank, in place in
     // pos_of_pair).
@@ -484,6 +500,45 @@ __global__ __launch_bounds__(kGroupThreads) void moe_place_kernel(
             pos_of_pair[p] = pos;
             src_token[pos] = p / top_k;
         }
+    }
+}
+
+// moe_rank_kernel and moe_place_kernel in one workgroup, for at most kChunk
+// pairs (one chunk): the same ranks, positions and tile table with one launch
+// less.  Latency bound: a few barriers and dependent loads.  171 pairs, 257
+// experts: one kernel of 7.5 us in place of two of 6 and 7.
+__global__ __launch_bounds__(kChunk) void moe_group_kernel(
+    const int* __restrict__ ids, int P, int experts, int bm, int top_k, int* __restrict__ tile_expert,
+    int* __restrict__ tile_start, int* __restrict__ tile_count, int* __restrict__ ntiles, int* __restrict__ nvalid,
+    int* __restrict__ pos_of_pair, int* __restrict__ src_token) {
+    constexpr int kWaves = kChunk / kWave;
+    __shared__ int wave_count[kWaves][kRouterMaxExperts];
+    __shared__ int buf[kWaves];
+    __shared__ int base[kRouterMaxExperts];
+    for (int i = threadIdx.x; i < kWaves * experts; i += kChunk) wave_count[i / experts][i % experts] = 0;
+    const int p = threadIdx.x;
+    const int e = p < P ? ids[p] : -1;
+    __syncthreads();
+    const int rank_in_wave = wave_rank(e, experts, wave_count[p / kWave]);
+    __syncthreads();
+    int total = 0;
+    if (p < experts) {
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            const int c = wave_count[w][p];
+            wave_count[w][p] = total;
+            total += c;
+        }
+    }
+    const int start = block_exclusive_scan(total, buf);
+    if (p < experts) base[p] = start;
+    write_tiles(total, start, bm, buf, tile_expert, tile_start, tile_count, ntiles, nvalid);
+    __syncthreads();
+    if (p < P) {
+        const bool valid = e >= 0 && e < experts;
+        const int pos = valid ? base[e] + wave_count[p / kWave][e] + rank_in_wave : -1;
+        pos_of_pair[p] = pos;
+        if (valid) src_token[pos] = p / top_k;
     }
 }
 
@@ -964,14 +1019,20 @@ int moe_grouped(const uint8_t* gate_up, const uint8_t* down, int experts, int H,
     const int thin = dwords ? L.thin : 0;
     const bool aligned16 = aligned(gate_up, 16) && aligned(down, 16) && shared_aligned(16);
 
-    int* chunk_counts = reinterpret_cast<int*>(ws + L.chunk_counts);
-    hipLaunchKernelGGL(moe_rank_kernel, dim3(L.chunks), dim3(kChunk), 0, stream, ids, P, experts, chunk_counts,
-                       pos_of_pair);
-    int status = launch_status();
-    if (status != Q3X_HIP_OK) return status;
-    hipLaunchKernelGGL(moe_place_kernel, dim3(L.chunks), dim3(kGroupThreads), 0, stream,
-                       static_cast<const int*>(chunk_counts), L.chunks, experts, thin ? thin : kWideBM, tile_expert, tile_start,
-                       tile_count, ntiles, nvalid, ids, P, top_k, pos_of_pair, src_token);
+    const int bm = thin ? thin : kWideBM;
+    int status;
+    if (L.chunks == 1) {
+        hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(kChunk), 0, stream, ids, P, experts, bm, top_k, tile_expert,
+                           tile_start, tile_count, ntiles, nvalid, pos_of_pair, src_token);
+    } else {
+        int* chunk_counts = reinterpret_cast<int*>(ws + L.chunk_counts);
+        hipLaunchKernelGGL(moe_rank_kernel, dim3(L.chunks), dim3(kChunk), 0, stream, ids, P, experts, chunk_counts,
+                           pos_of_pair);
+        if ((status = launch_status()) != Q3X_HIP_OK) return status;
+        hipLaunchKernelGGL(moe_place_kernel, dim3(L.chunks), dim3(kGroupThreads), 0, stream,
+                           static_cast<const int*>(chunk_counts), L.chunks, experts, bm, tile_expert, tile_start,
+                           tile_count, ntiles, nvalid, ids, P, top_k, pos_of_pair, src_token);
+    }
     if ((status = launch_status()) != Q3X_HIP_OK) return status;
 
     const int tiles_bound = L.max_tiles;
@@ -1030,8 +1091,12 @@ int moe_grouped(const uint8_t* gate_up, const uint8_t* down, int experts, int H,
 // experts' matvec stages it -- same sum order, same products -- so router
 // and experts see identical normalised values), and the row's dot reads x
 // from there.  Rows and x 16-byte aligned, H % 32 == 0, x within
-// router_gemv_lds_bytes.
+// router_gemv_lds_bytes.  blockIdx.y: the token; up to kRouterGemvTokens
+// of them each token's workgroups read the router's rows again from L2 (19
+// tokens, 256 experts, H = 2048: 5.5 us, where the split GEMM and its fixup
+// took 14).
 constexpr int kRouterHeld = 8;
+constexpr int kRouterGemvTokens = 32;
 inline size_t router_gemv_lds_bytes(int H) { return pipe_x_bytes(H / kBlock) + 64; }
 
 template <class In>
@@ -1044,6 +1109,8 @@ __global__ __launch_bounds__(256) void router_gemv_bf16_kernel(const uint16_t* _
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
     const int r = blockIdx.x * 4 + wave;  // rows past the gate row read zeros and store nothing
+    const size_t token = blockIdx.y;
+    x += token * H;
     const int bpr = H / kBlock;
     const uint16_t* row = r < experts ? router + static_cast<size_t>(r) * H : gate_row;
     // A buffer resource of the row's bytes: zeros past its end (and for rows
@@ -1080,8 +1147,8 @@ __global__ __launch_bounds__(256) void router_gemv_bf16_kernel(const uint16_t* _
         step(c, __builtin_amdgcn_raw_buffer_load_b128(rr, 2 * c, 0, 0));
     const float total = group_sum<kWave>(acc);
     if (lane == 0 && r <= experts) {
-        if (r < experts) logits[r] = total;
-        else *gate_logit = total;
+        if (r < experts) logits[token * experts + r] = total;
+        else gate_logit[token] = total;
     }
 }
 
@@ -1269,10 +1336,10 @@ int moe_layer_run(const q3x_hip_moe_layer_weights& w, const float* X, int tokens
     int status;
 
     // Router logits and the shared expert's gate logit.
-    if (tokens == 1 && router_gemv_lds_bytes(H) <= 64 * 1024) {
+    if (tokens <= kRouterGemvTokens && router_gemv_lds_bytes(H) <= 64 * 1024) {
         const auto* rows = reinterpret_cast<const uint16_t*>(router);
         const auto* grow = reinterpret_cast<const uint16_t*>(gate_row);
-        const dim3 grid((E + 1 + 3) / 4);
+        const dim3 grid((E + 1 + 3) / 4, tokens);
         if (norm_w)
             hipLaunchKernelGGL(router_gemv_bf16_kernel<NormInput>, grid, dim3(256), router_gemv_lds_bytes(H), stream,
                                rows, grow, E, H, X, NormInput{norm_w}, logits, gate);

@@ -10,6 +10,7 @@ import pytest
 import oracle
 import qwen3x_amd as q3x
 from tests.helpers import Q4_0, Q8_0, dequant_numpy, random_blocks, row_bound
+from tests import test_gpu_moe_layer as layers
 from tests.test_gpu_parity import _torch, dev, host, moe_bound, say
 
 pytestmark = pytest.mark.gpu
@@ -115,3 +116,12 @@ def test_few_pair_experts(type_, E, k, tokens, H, I):
         assert np.all(np.abs(got[0] - want) <= bound)
         # The two tile shapes: the same exact products in FP32 sums of another order.
         assert np.all(np.abs(got[0].astype(np.float64) - got[1]) <= 2 * bound)
+
+
+@pytest.mark.parametrize("type_", [Q8_0, Q4_0])
+@pytest.mark.parametrize("E,k,H,I,SI,tokens", [
+    (64, 4, 256, 96, 96, 2), (64, 4, 256, 96, 64, 32), (64, 4, 256, 96, 96, 33),  # the per-token router's last count
+    (40, 3, 128, 32, 32, 256), (40, 3, 128, 32, 32, 257),  # 1024 and 1028 pairs: one grouping workgroup and two
+    (1023, 2, 64, 32, 32, 20), (1024, 2, 64, 64, 32, 20)])
+def test_few_token_layer_routing(type_, E, k, H, I, SI, tokens):
+    layers.test_moe_layer_parity(type_, E, H, I, SI, k, tokens)
