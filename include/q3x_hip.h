@@ -103,8 +103,9 @@ int q3x_hip_gemm(const void* w, uint32_t type, int rows, int cols,
  * same shape and arguments as q3x_hip_gemm, with a workspace of at least
  * q3x_hip_gemm_workspace_bytes(type, rows, cols, count) bytes (16-byte
  * aligned; smaller or null runs q3x_hip_gemm's launch): a launch of few
- * output tiles over a long K (e.g. 512 tokens x 5120 rows x 17408 columns)
- * then fills the chip, each tile's K ranges summed by a second launch in K
+ * output tiles over a long K (e.g. 512 tokens x 5120 rows x 17408 columns),
+ * or the last, short round of one of a few more tiles than the chip runs at
+ * once (512 x 17408 x 5120), then fills the chip, each tile's K ranges summed by a second launch in K
  * order.  Deterministic; the sums run in another order than q3x_hip_gemm's,
  * within the same tolerance against the reference.  The workspace holds the
  * partial sums from the first launch to the second, so calls that share one

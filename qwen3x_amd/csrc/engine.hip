@@ -1835,7 +1835,8 @@ int enqueue(q3x_hip_engine& e, int count, bool logits) {
                                    L.post_norm, c.H, e.normalized);
                 // A chunk: gate and up as one GEMM with the SwiGLU in its
                 // epilogue (one pass over h instead of three).
-                rc = count > 1 ? gate_up_swiglu(L.gate.w, L.up.w, type, c.I, c.H, e.normalized, count, e.ffn_gate, s)
+                rc = count > 1 ? gate_up_swiglu(L.gate.w, L.up.w, type, c.I, c.H, e.normalized, count, e.ffn_gate,
+                                                gemm_ws.p, gemm_ws.bytes, s)
                                : Q3X_HIP_ENOTSUP;
                 swiglu_done = rc == Q3X_HIP_OK;
                 if (rc == Q3X_HIP_ENOTSUP) rc = apply_group(gate_up, ffn, 2, type, c.H, e.normalized, count, s, gemm_ws);
@@ -2017,6 +2018,10 @@ extern "C" int q3x_hip_engine_create(const q3x_hip_model_config* config, const v
         for (const LayerWeights& L : e->layers)
             for (const Mat* m : {&L.qkv, &L.z, &L.a, &L.b, &L.out, &L.q, &L.k, &L.v, &L.o, &L.gate, &L.up, &L.down})
                 e->gemm_ws_bytes = std::max(e->gemm_ws_bytes, need(*m));
+        if (!c.experts)  // the paired gate and up GEMM of the dense FFNs
+            for (size_t n = 64; n < R + 64; n += 64)
+                e->gemm_ws_bytes = std::max(
+                    e->gemm_ws_bytes, gate_up_swiglu_workspace_bytes(c.I, c.H, static_cast<int>(std::min(n, R))));
         if (e->gemm_ws_bytes > kGemmScratchMax) e->gemm_ws_bytes = kGemmScratchMax;
     }
     // One arena: the work rows of a chunk, the recurrent state and its

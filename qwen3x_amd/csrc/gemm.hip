@@ -26,7 +26,8 @@ struct DenseGemm {
     float* Y;
     int rows;
     bool accumulate;
-    int ksplit = 1;         // units per tile over K (set by the launch)
+    int kwhole = 0;         // tiles before the split ones that run whole, and
+    int ksplit = 1;         // units per tile over K after them (set by the launch)
     float* part = nullptr;  // their partial sums (caller's workspace)
     __device__ bool tile(int ty, int bm, GemmTile& t) const {
         t.m0 = ty * bm;
@@ -84,7 +85,7 @@ int gemm(const void* w, uint32_t type, int rows, int cols, const float* X, int c
     // aligned); otherwise q3x_hip_gemm's plan.
     const size_t need = x3_plan(rows, count, cols, false, SIZE_MAX).workspace_bytes();
     const size_t usable = need > 0 && aligned(workspace, 16) && workspace_bytes >= need ? need : 0;
-    DenseGemm g{0, X, cols, count, static_cast<const uint8_t*>(w), row_bytes, Y, rows, accumulate != 0, 1,
+    DenseGemm g{0, X, cols, count, static_cast<const uint8_t*>(w), row_bytes, Y, rows, accumulate != 0, 0, 1,
                 static_cast<float*>(workspace)};
     return type == Q3X_HIP_MATRIX_Q8_0 ? launch_x3<Q3X_HIP_MATRIX_Q8_0>(g, rows, count, cols, stream, usable)
                                        : launch_x3<Q3X_HIP_MATRIX_Q4_0>(g, rows, count, cols, stream, usable);

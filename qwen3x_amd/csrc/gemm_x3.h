@@ -80,21 +80,26 @@ __device__ __forceinline__ void split3(float a, uint32_t& h1, uint32_t& h2, uint
     h3 = __float_as_uint(r - __uint_as_float(h2));
 }
 
-// K split over workgroups (policies with ksplit and part members, e.g. a
-// GEMM given a workspace): the launch has ksplit units per tile, unit s
+// K split over workgroups (policies with kwhole, ksplit and part members,
+// e.g. a GEMM given a workspace): the launch's first kwhole tiles run whole
+// and each tile after them as ksplit units, unit s
 // taking the tile's K blocks [s * per, (s + 1) * per), per = ceil(blocks /
 // ksplit); each unit writes its sums, as its threads hold them, to its slot
 // of `part`, and gemm_x3_fixup_kernel adds a tile's units in K order and
 // stores.  So a launch of few tiles over long K (512 tokens x 5120 rows x
-// 17408 columns is 80 tiles of 128 x 256 for 256 CUs) fills the chip;
-// results are deterministic, their sums in another order than unsplit.
+// 17408 columns is 80 tiles of 128 x 256 for 256 CUs) fills the chip, and a
+// launch of some more tiles than CUs (272 for 512 x 17408 x 5120) splits
+// only the last, short round; results are deterministic, their sums in
+// another order than unsplit.
 template <class P, class = void>
 struct KSplit {
+    __device__ static int whole(const P&) { return 0; }
     __device__ static int count(const P&) { return 1; }
     __device__ static float* part(const P&) { return nullptr; }
 };
 template <class P>
 struct KSplit<P, decltype(void(std::declval<const P&>().ksplit))> {
+    __device__ static int whole(const P& p) { return p.kwhole; }
     __device__ static int count(const P& p) { return p.ksplit; }
     __device__ static float* part(const P& p) { return p.part; }
 };
@@ -177,12 +182,23 @@ __global__ __launch_bounds__(KS * WM * WN * kWave) void gemm_x3_kernel(Policy po
     };
 
     // Units of a split launch are numbered split-major (unit = split *
-    // tiles + tile), so an XCD's contiguous run shares its A tile's K range.
-    const int S = KSplit<Policy>::count(pol);
-    int bx = blockIdx.x, by = blockIdx.y, split = 0, tile_id = 0;
+    // tiles + tile), so an XCD's contiguous run shares its A tile's K range;
+    // the whole tiles (a multiple of kXcds) come first, with a remap of
+    // their own.
+    const int whole = KSplit<Policy>::whole(pol);
+    int S = KSplit<Policy>::count(pol);
+    int bx = blockIdx.x, by = blockIdx.y, split = 0, slot_id = 0;
     if constexpr (Policy::kLinearGrid) {
-        const int total = LinearTotal<Policy>::get(pol, gridDim.x), L = blockIdx.x;
+        int total = LinearTotal<Policy>::get(pol, gridDim.x), L = blockIdx.x, first = 0;
         if (L >= total) return;
+        if (L < whole) {
+            total = whole;
+            S = 1;
+        } else {
+            total -= whole;
+            L -= whole;
+            first = whole;
+        }
         const int q = total / kXcds, r = total % kXcds, xcd = L % kXcds, k = L / kXcds;
         int t = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + k;
         if (S > 1) {
@@ -190,7 +206,8 @@ __global__ __launch_bounds__(KS * WM * WN * kWave) void gemm_x3_kernel(Policy po
             split = t / tiles;
             t %= tiles;
         }
-        tile_id = t;
+        slot_id = t;
+        t += first;
         bx = t % pol.tiles_x;
         by = t / pol.tiles_x;
     }
@@ -380,7 +397,7 @@ __global__ __launch_bounds__(KS * WM * WN * kWave) void gemm_x3_kernel(Policy po
         // This unit's sums to its slot (coalesced: value v of thread t at
         // v * NT + t); the fixup adds the tile's units and stores.
         float* slot = KSplit<Policy>::part(pol) +
-                      (static_cast<size_t>(tile_id) * S + split) * x3_unit_floats<WM, WN, SM, SN>();
+                      (static_cast<size_t>(slot_id) * S + split) * x3_unit_floats<WM, WN, SM, SN>();
 #pragma unroll
         for (int i = 0; i < SM; ++i)
 #pragma unroll
@@ -393,7 +410,7 @@ __global__ __launch_bounds__(KS * WM * WN * kWave) void gemm_x3_kernel(Policy po
 }
 
 // The stores of a split launch, one output value per thread: value f (in
-// the units' layout, f = v * NT + t for value v of thread t) of tile
+// the units' layout, f = v * NT + t for value v of thread t) of split tile
 // blockIdx.x / (BM * BN / 256), its units added in K order (unit 0 first),
 // stored where gemm_x3_kernel's thread t would store its value v.  With
 // kPairedColumns the thread of an even column block stores the pair, its
@@ -406,12 +423,12 @@ __global__ __launch_bounds__(256) void gemm_x3_fixup_kernel(Policy pol, int rows
     constexpr int U = static_cast<int>(x3_unit_floats<WM, WN, SM, SN>());  // BM * BN
     static_assert(U % 256 == 0, "whole workgroups per tile");
     constexpr int kPerTile = U / 256;
-    const int t = blockIdx.x / kPerTile;
+    const int slot = blockIdx.x / kPerTile, t = pol.kwhole + slot;
     const int f = (blockIdx.x % kPerTile) * 256 + threadIdx.x;
     GemmTile tile;
     if (!pol.tile(t / pol.tiles_x, BM, tile)) return;
     const int S = pol.ksplit;
-    const float* units = pol.part + static_cast<size_t>(t) * S * U;
+    const float* units = pol.part + static_cast<size_t>(slot) * S * U;
     auto unit_sum = [&](int g) {
         float sum = units[g];
         for (int u = 1; u < S; ++u) sum += units[static_cast<size_t>(u) * U + g];
@@ -438,8 +455,7 @@ __global__ __launch_bounds__(256) void gemm_x3_fixup_kernel(Policy pol, int rows
 // on 8 waves of 32x32 (three), 64 x 64 on 4 waves of 32x32 (four).  128 x 192
 // exists for row counts that 256 leaves uneven over the CUs: 512 tokens x
 // 12288 rows x 4096 columns is 256 tiles of it, one per CU, at 306 TFLOP/s
-// (Q8_0; 260 on 128 x 256, whose 192 tiles leave 64 CUs idle), and 512 x
-// 17408 x 5120 runs at 257 (238 on 64 x 128); with many tiles per CU it
+// (Q8_0; 260 on 128 x 256, whose 192 tiles leave 64 CUs idle); with many tiles per CU it
 // runs at ~340, below 128 x 256's ~383.  Over long K (>= kX3LongK) a
 // 64 x 128 tile can also run on two halves of 8 waves, each over half the
 // K blocks with its own LDS buffers, the second half's sums added to the
@@ -453,8 +469,7 @@ __global__ __launch_bounds__(256) void gemm_x3_fixup_kernel(Policy pol, int rows
 // a time, and a CU holding k of them runs at the shape's measured rate for
 // k (TFLOP/s over the chip, MI355X, dense Q8_0/Q4_0).  Measured, e.g.: 4096
 // tokens x 12288 rows x 4096 columns 370 TFLOP/s on 128 x 256; 512 x 4096
-// x 12288 (64 tiles of 128 x 256) 208 on 64 x 128; 512 x 17408 x 5120 253
-// on 64 x 128 (272 tiles of 128 x 256 would leave 16 CUs a second one).
+// x 12288 (64 tiles of 128 x 256) 208 on 64 x 128.
 enum class X3Shape { k128x256, k64x128, k64x64, k128x192, k64x128_split };
 
 // Per-CU time of `tiles` tiles (or units) of `area` outputs each (in units
@@ -474,13 +489,17 @@ inline double x3_estimate(long long tiles, double area, int occupancy, const dou
 // 512 tokens x 12288- and 17408-column matrices, a few % slower on short K).
 constexpr int kX3LongK = 8192;
 
-// A launch: the tile shape and the units per tile of a K split (1: none).
+// A launch: the tile shape, the units per tile of a K split (1: none) and the
+// tiles before the split ones that run whole.
 struct X3Plan {
     X3Shape shape;
     int split;
     long long tiles;
     int bm, bn;
-    size_t workspace_bytes() const { return split > 1 ? static_cast<size_t>(tiles) * split * bm * bn * 4 : 0; }
+    long long whole = 0;
+    size_t workspace_bytes() const {
+        return split > 1 ? static_cast<size_t>(tiles - whole) * split * bm * bn * 4 : 0;
+    }
 };
 
 // The plan of least estimated time for rows weight rows, count A rows and
@@ -522,28 +541,45 @@ inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspa
     constexpr double kRoundSeconds = 3e-6, kRoundSecondsShared = 2e-6;
     constexpr double kFixupBytesPerSecond = 2e12;
     constexpr double kLaunchSeconds = 5e-6;
-    constexpr int kSplits[] = {1, 2, 3, 4, 6, 8};
+    constexpr int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
+    constexpr int kMostSplit = 8, kTailUnits = 2 * kCUs;
     X3Plan best{X3Shape::k128x256, 1, 0, 128, 256};
     double best_t = 1e300;
     for (const Option& o : options) {
         if (!o.ok) continue;
         const long long t = tiles(o.bm, o.bn);
         const double area = static_cast<double>(o.bm) * o.bn;
-        for (const int split : kSplits) {
-            const int per = (blocks + split - 1) / split;
-            if (split > 1 && (per < 8 || (split - 1) * per >= blocks)) continue;
-            const X3Plan plan{o.shape, split, t, o.bm, o.bn};
-            if (plan.workspace_bytes() > workspace) continue;
-            double sec = x3_estimate(t * split, area / split, o.occupancy, o.rate) * 2.0 * cols * kCUs / 1e12;
-            if (split > 1) {
-                const long long rounds = (t * split + static_cast<long long>(kCUs) * o.occupancy - 1) /
-                                         (static_cast<long long>(kCUs) * o.occupancy);
-                sec += rounds * (o.occupancy == 1 ? kRoundSeconds : kRoundSecondsShared) + kLaunchSeconds +
-                       static_cast<double>(t) * area * 4.0 * (split + 1) / kFixupBytesPerSecond;
-            }
-            if (sec < best_t) {
-                best_t = sec;
-                best = plan;
+        const double unit = 2.0 * cols * kCUs / 1e12;  // seconds of area / rate
+        // The tiles of the full rounds, where a short round follows them: the
+        // one-per-CU shapes may split that round's tiles alone, to at most
+        // two units per CU (64 MiB of sums).  Measured with the best plan
+        // before (us, Q8_0): 512 x 17408 x 5120, 272 tiles, 16 of them split
+        // in 16: 310 -> 252 (362 TFLOP/s); 512 x 24576 x 4096: 314 -> 286;
+        // 1024 x 17408 x 5120: 567 -> 486; 2048 x 5120 x 4096: 334 -> 241;
+        // 4096 x 5120 x 12288: 1465 -> 1395.  Over 200 shapes of 256 to 4096
+        // tokens x 4096 to 24576 rows no choice was slower than before.
+        const long long rounds = t / kCUs * kCUs;
+        const bool tail = o.occupancy == 1 && rounds > 0 && rounds < t;
+        for (const long long whole : {0LL, tail ? rounds : 0LL}) {
+            const long long part = t - whole;
+            for (const int split : kSplits) {
+                const int per = (blocks + split - 1) / split;
+                if (split > 1 && (per < 8 || (split - 1) * per >= blocks)) continue;
+                if (whole > 0 ? split == 1 || part * split > kTailUnits : split > kMostSplit) continue;
+                const X3Plan plan{o.shape, split, t, o.bm, o.bn, whole};
+                if (plan.workspace_bytes() > workspace) continue;
+                double sec = (x3_estimate(whole, area, o.occupancy, o.rate) +
+                              x3_estimate(part * split, area / split, o.occupancy, o.rate)) * unit;
+                if (split > 1) {
+                    const long long more = (part * split + static_cast<long long>(kCUs) * o.occupancy - 1) /
+                                           (static_cast<long long>(kCUs) * o.occupancy);
+                    sec += more * (o.occupancy == 1 ? kRoundSeconds : kRoundSecondsShared) + kLaunchSeconds +
+                           static_cast<double>(part) * area * 4.0 * (split + 1) / kFixupBytesPerSecond;
+                }
+                if (sec < best_t) {
+                    best_t = sec;
+                    best = plan;
+                }
             }
         }
     }
@@ -563,20 +599,22 @@ struct HasKSplit<P, decltype(void(std::declval<P&>().ksplit))> : std::true_type 
 // weight rows, on a 1-D grid (Policy::kLinearGrid) of all tiles (units);
 // with split > 1 (policies with a workspace), the fixup launch follows.
 template <uint32_t QT, int WM, int WN, int SM, int SN, int PF, bool CF, class P, int KS = 1>
-int launch_x3_tiles(P pol, int rows, int count, int cols, hipStream_t stream, int split = 1) {
+int launch_x3_tiles(P pol, int rows, int count, int cols, hipStream_t stream, int split = 1, long long whole = 0) {
     constexpr int BM = WM * SM * 16, BN = WN * SN * 16;
     pol.tiles_x = (rows + BN - 1) / BN;
     const long long tiles = static_cast<long long>(pol.tiles_x) * ((count + BM - 1) / BM);
-    if (tiles * split > 0x7fffffffLL || (split > 1 && tiles * (BM * BN / 256) > 0x7fffffffLL))
-        return Q3X_HIP_EINVAL;
+    const long long parted = tiles - whole;
+    const long long units = whole + parted * split;
+    if (units > 0x7fffffffLL || (split > 1 && parted * (BM * BN / 256) > 0x7fffffffLL)) return Q3X_HIP_EINVAL;
     if constexpr (HasKSplit<P>::value) {
         if (split > 1 && pol.part == nullptr) return Q3X_HIP_EINVAL;  // the units' sums need a workspace
         pol.ksplit = split;
+        pol.kwhole = static_cast<int>(whole);
     } else if (split != 1) {
         return Q3X_HIP_EINVAL;
     }
     hipLaunchKernelGGL((gemm_x3_kernel<QT, WM, WN, SM, SN, P, PF, CF, KS>),
-                       dim3(static_cast<unsigned>(tiles * split)), dim3(KS * WM * WN * kWave), 0, stream, pol, rows,
+                       dim3(static_cast<unsigned>(units)), dim3(KS * WM * WN * kWave), 0, stream, pol, rows,
                        cols);
     if constexpr (HasKSplit<P>::value) {
         if (split > 1) {
@@ -584,7 +622,7 @@ int launch_x3_tiles(P pol, int rows, int count, int cols, hipStream_t stream, in
             if (status != Q3X_HIP_OK) return status;
             constexpr int kPerTile = BM * BN / 256;
             hipLaunchKernelGGL((gemm_x3_fixup_kernel<WM, WN, SM, SN, P>),
-                               dim3(static_cast<unsigned>(tiles * kPerTile)), dim3(256), 0, stream, pol, rows);
+                               dim3(static_cast<unsigned>(parted * kPerTile)), dim3(256), 0, stream, pol, rows);
         }
     }
     return launch_status();
@@ -600,14 +638,14 @@ int launch_x3(const P& pol, int rows, int count, int cols, hipStream_t stream, s
         // The one-per-CU shapes with two stages of loads ahead: 1-3% faster
         // than one (and than compute-first) at 512-4096 tokens.
         case X3Shape::k128x256:
-            return launch_x3_tiles<QT, 2, 4, 4, 4, 2, false>(pol, rows, count, cols, stream, split);
+            return launch_x3_tiles<QT, 2, 4, 4, 4, 2, false>(pol, rows, count, cols, stream, split, plan.whole);
         case X3Shape::k128x192:
             if constexpr (!P::kPairedColumns)
-                return launch_x3_tiles<QT, 2, 4, 4, 3, 2, false>(pol, rows, count, cols, stream, split);
+                return launch_x3_tiles<QT, 2, 4, 4, 3, 2, false>(pol, rows, count, cols, stream, split, plan.whole);
             else
-                return launch_x3_tiles<QT, 2, 4, 4, 4, 2, false>(pol, rows, count, cols, stream, split);
+                return launch_x3_tiles<QT, 2, 4, 4, 4, 2, false>(pol, rows, count, cols, stream, split, plan.whole);
         case X3Shape::k64x128_split:
-            return launch_x3_tiles<QT, 2, 4, 2, 2, 1, false, P, 2>(pol, rows, count, cols, stream, split);
+            return launch_x3_tiles<QT, 2, 4, 2, 2, 1, false, P, 2>(pol, rows, count, cols, stream, split, plan.whole);
         case X3Shape::k64x128:
             if (cols >= kX3LongK)
                 return launch_x3_tiles<QT, 2, 4, 2, 2, 2, false>(pol, rows, count, cols, stream, split);

@@ -23,8 +23,12 @@ int moe_layer_decode_add(const q3x_hip_moe_layer_weights& layer, const float* X,
 // one 32-column tile -- each product summed as the GEMM launches sum it
 // (K in block order within one half), then silu(g) * u as swiglu_kernel.
 // Q3X_HIP_ENOTSUP (nothing enqueued) where I % 64 != 0 or an operand is
-// unaligned (weights 2, X 16, h 4 bytes).
+// unaligned (weights 2, X 16, h 4 bytes).  With a workspace (null, or 16-byte
+// aligned) the launch may split K, as q3x_hip_gemm_ws does:
+// gate_up_swiglu_workspace_bytes is what its plan asks for, and with less it
+// takes the best plan that fits.
+size_t gate_up_swiglu_workspace_bytes(int I, int H, int count);
 int gate_up_swiglu(const void* gate, const void* up, uint32_t type, int I, int H, const float* X, int count,
-                   float* h, hipStream_t stream);
+                   float* h, void* workspace, size_t workspace_bytes, hipStream_t stream);
 
 }  // namespace q3x

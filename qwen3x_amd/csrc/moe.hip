@@ -1164,7 +1164,8 @@ struct TokenTiles {
     const float* X;
     int cols;
     int count;
-    int ksplit = 1;         // units per tile over K (set by the launch)
+    int kwhole = 0;         // tiles before the split ones that run whole, and
+    int ksplit = 1;         // units per tile over K after them (set by the launch)
     float* part = nullptr;  // their partial sums
     __device__ bool tile(int ty, int bm, GemmTile& t) const {
         t.m0 = ty * bm;
@@ -1553,8 +1554,12 @@ extern "C" int q3x_hip_moe_layer(const q3x_hip_moe_layer_weights* layer, const f
     return moe_layer_checked(layer, X, tokens, Y, ids, weights, workspace, workspace_bytes, stream, false);
 }
 
+size_t q3x::gate_up_swiglu_workspace_bytes(int I, int H, int count) {
+    return I % 64 == 0 ? token_gemm_part_bytes(2 * I, count, H, true) : 0;
+}
+
 int q3x::gate_up_swiglu(const void* gate, const void* up, uint32_t type, int I, int H, const float* X, int count,
-                        float* h, hipStream_t stream) {
+                        float* h, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     size_t bytes;
     if (!is_quant_type(type) || count <= 0 || I % 64 != 0 || !quantized_size(type, I, H, &bytes))
         return Q3X_HIP_ENOTSUP;
@@ -1567,8 +1572,10 @@ int q3x::gate_up_swiglu(const void* gate, const void* up, uint32_t type, int I, 
     if (thin_ok(count, 2 * I, H, aligned(gate, 4) && aligned(up, 4)))
         return type == Q3X_HIP_MATRIX_Q8_0 ? launch_thin<Q3X_HIP_MATRIX_Q8_0>(g, 2 * I, count, H, aligned16, stream)
                                            : launch_thin<Q3X_HIP_MATRIX_Q4_0>(g, 2 * I, count, H, aligned16, stream);
-    return type == Q3X_HIP_MATRIX_Q8_0 ? launch_token_gemm<Q3X_HIP_MATRIX_Q8_0>(g, 2 * I, stream)
-                                       : launch_token_gemm<Q3X_HIP_MATRIX_Q4_0>(g, 2 * I, stream);
+    float* const part = aligned(workspace, 16) ? static_cast<float*>(workspace) : nullptr;
+    return type == Q3X_HIP_MATRIX_Q8_0
+               ? launch_token_gemm<Q3X_HIP_MATRIX_Q8_0>(g, 2 * I, stream, part, workspace_bytes)
+               : launch_token_gemm<Q3X_HIP_MATRIX_Q4_0>(g, 2 * I, stream, part, workspace_bytes);
 }
 
 int q3x::moe_layer_decode_add(const q3x_hip_moe_layer_weights& layer, const float* X, const uint16_t* norm_w,
