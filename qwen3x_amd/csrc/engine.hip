@@ -30,7 +30,9 @@
 
 #include <algorithm>
 #include <new>
+#include <set>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "common.h"
@@ -2004,12 +2006,14 @@ extern "C" int q3x_hip_engine_create(const q3x_hip_model_config* config, const v
         e->delta_ws_floats = (R + kDeltaChunk - 1) / kDeltaChunk * c.VH * static_cast<size_t>(kDeltaChunkFloats);
     // The prefill GEMMs' K splits: the most any of the chunk's GEMMs asks
     // for at any row count up to a chunk (a call given less runs unsplit),
-    // within kGemmScratchMax.
+    // within kGemmScratchMax.  Every tile height is a multiple of 16, so the
+    // plans change there only; matrices of one shape ask once.
     if (R > 1) {
+        std::set<std::pair<int, int>> asked;
         auto need = [&](const Mat& m) {
             size_t most = 0;
-            if (!m.w) return most;
-            for (size_t n = 64; n < R + 64; n += 64) {
+            if (!m.w || !asked.emplace(m.rows, m.cols).second) return most;
+            for (size_t n = 16; n < R + 16; n += 16) {
                 const int count = static_cast<int>(std::min(n, R));
                 most = std::max(most, q3x_hip_gemm_workspace_bytes(c.matrix_type, m.rows, m.cols, count));
             }
@@ -2019,7 +2023,7 @@ extern "C" int q3x_hip_engine_create(const q3x_hip_model_config* config, const v
             for (const Mat* m : {&L.qkv, &L.z, &L.a, &L.b, &L.out, &L.q, &L.k, &L.v, &L.o, &L.gate, &L.up, &L.down})
                 e->gemm_ws_bytes = std::max(e->gemm_ws_bytes, need(*m));
         if (!c.experts)  // the paired gate and up GEMM of the dense FFNs
-            for (size_t n = 64; n < R + 64; n += 64)
+            for (size_t n = 16; n < R + 16; n += 16)
                 e->gemm_ws_bytes = std::max(
                     e->gemm_ws_bytes, gate_up_swiglu_workspace_bytes(c.I, c.H, static_cast<int>(std::min(n, R))));
         if (e->gemm_ws_bytes > kGemmScratchMax) e->gemm_ws_bytes = kGemmScratchMax;

@@ -83,12 +83,12 @@ int gemm(const void* w, uint32_t type, int rows, int cols, const float* X, int c
     }
     // The split plan runs only with all of the workspace it asks for (16-byte
     // aligned); otherwise q3x_hip_gemm's plan.
-    const size_t need = x3_plan(rows, count, cols, false, SIZE_MAX).workspace_bytes();
+    const size_t need = x3_plan(rows, count, cols, false, SIZE_MAX, true).workspace_bytes();
     const size_t usable = need > 0 && aligned(workspace, 16) && workspace_bytes >= need ? need : 0;
     DenseGemm g{0, X, cols, count, static_cast<const uint8_t*>(w), row_bytes, Y, rows, accumulate != 0, 0, 1,
                 static_cast<float*>(workspace)};
-    return type == Q3X_HIP_MATRIX_Q8_0 ? launch_x3<Q3X_HIP_MATRIX_Q8_0>(g, rows, count, cols, stream, usable)
-                                       : launch_x3<Q3X_HIP_MATRIX_Q4_0>(g, rows, count, cols, stream, usable);
+    return type == Q3X_HIP_MATRIX_Q8_0 ? launch_x3<Q3X_HIP_MATRIX_Q8_0, true>(g, rows, count, cols, stream, usable)
+                                       : launch_x3<Q3X_HIP_MATRIX_Q4_0, true>(g, rows, count, cols, stream, usable);
 }
 
 }  // namespace
@@ -101,7 +101,7 @@ extern "C" int q3x_hip_gemm(const void* w, uint32_t type, int rows, int cols, co
 extern "C" size_t q3x_hip_gemm_workspace_bytes(uint32_t type, int rows, int cols, int count) {
     size_t bytes;
     if (type == Q3X_HIP_MATRIX_BF16 || count <= 0 || !quantized_size(type, rows, cols, &bytes)) return 0;
-    return x3_plan(rows, count, cols, false, SIZE_MAX).workspace_bytes();
+    return x3_plan(rows, count, cols, false, SIZE_MAX, true).workspace_bytes();
 }
 
 extern "C" int q3x_hip_gemm_ws(const void* w, uint32_t type, int rows, int cols, const float* X, int count,

@@ -470,7 +470,17 @@ __global__ __launch_bounds__(256) void gemm_x3_fixup_kernel(Policy pol, int rows
 // k (TFLOP/s over the chip, MI355X, dense Q8_0/Q4_0).  Measured, e.g.: 4096
 // tokens x 12288 rows x 4096 columns 370 TFLOP/s on 128 x 256; 512 x 4096
 // x 12288 (64 tiles of 128 x 256) 208 on 64 x 128.
-enum class X3Shape { k128x256, k64x128, k64x64, k128x192, k64x128_split };
+//
+// 48 x 128 (4 waves of 48x32, four workgroups per CU), 80 x 256 (8 waves of
+// 80x32, two) and 96 x 256 (8 waves of 48x64, one) are for few A rows, where
+// the rows a tile is padded by are work done for nothing: see x3_plan's
+// `few`.
+enum class X3Shape { k128x256, k64x128, k64x64, k128x192, k64x128_split, k48x128, k80x256, k96x256 };
+
+// A rows up to which x3_plan's `few` adds the shapes for few A rows: two 96-row
+// tiles.  Past it the other shapes' padding is small, and 193 to 256 rows gained
+// nothing.
+constexpr int kX3FewRows = 192;
 
 // Per-CU time of `tiles` tiles (or units) of `area` outputs each (in units
 // of area / (TFLOP/s): multiply by 2 K 256 / 1e12 for seconds).
@@ -508,7 +518,19 @@ struct X3Plan {
 // rate, plus a per-round cost for its shorter pipeline (prologue, drain and
 // the partial-sum stores), and the launch adds the fixup: the units' sums
 // read back and the outputs written, and one more launch.
-inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspace) {
+//
+// few: with the shapes for few A rows (up to kX3FewRows).  A call of 77 rows
+// pays for 128 on the shapes above and one of 150 for 192 or 256; 80 x 256 and
+// 96 x 256 tiles hold them with 80 or 96 and 160 or 192 rows, 48 x 128 up to 48
+// (two of it lost to one 96 x 256).  Their K takes up to 16 splits: one A tile of
+// a 4096-row matrix is 16 to 32 tiles for 256 CUs.  The rates were fitted to a
+// sweep of every shape and split over 33 to 192 rows and 20 matrices (700 to
+// 20000 rows, 1024 to 24576 columns, Q8_0 and Q4_0); the plan's time there
+// against the one without these shapes, geometric means: 33-48 rows 0.89, 65-80
+// 0.84, 81-96 0.89, 129-160 0.87, 161-192 0.93, none slower by more than 3%
+// (49-64 and 97-128 rows keep the shapes above).  77 x 17408 x 5120 Q4_0 80.6
+// -> 65.0 us, 77 x 5120 x 17408 87.9 -> 61.5, 40 x 12288 x 4096 Q8_0 38.4 -> 32.7.
+inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspace, bool few = false) {
     auto tiles = [&](int bm, int bn) {
         return static_cast<long long>((rows + bn - 1) / bn) * ((count + bm - 1) / bm);
     };
@@ -518,19 +540,27 @@ inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspa
     static constexpr double r64[] = {150.0, 190.0, 215.0, 230.0};
     static constexpr double r192[] = {300.0};
     static constexpr double r64x128_split[] = {240.0};  // K halves on 16 waves, one workgroup per CU
+    static constexpr double r48[] = {132.0, 196.0, 180.0, 160.0};
+    static constexpr double r80[] = {267.0, 273.0};
+    static constexpr double r96[] = {300.0};
     struct Option {
         X3Shape shape;
         int bm, bn, occupancy;
         const double* rate;
         bool ok;
+        int most_split = 8;
     };
     const bool long_k = cols >= kX3LongK;
-    const Option options[5] = {
+    few = few && count <= kX3FewRows;
+    const Option options[8] = {
         {X3Shape::k128x256, 128, 256, 1, r256, true},
         {X3Shape::k64x128, 64, 128, 3, long_k ? r64x128_long : r64x128, true},
         {X3Shape::k64x64, 64, 64, 4, r64, true},
         {X3Shape::k128x192, 128, 192, 1, r192, !paired},
         {X3Shape::k64x128_split, 64, 128, 1, r64x128_split, long_k},
+        {X3Shape::k48x128, 48, 128, 4, r48, few && count <= 48, 16},
+        {X3Shape::k80x256, 80, 256, 2, r80, few, 16},
+        {X3Shape::k96x256, 96, 256, 1, r96, few, 16},
     };
     const int blocks = cols / kBlock;
     // Fitted to a sweep of every shape at splits 1, 2, 3, 4, 6 and 8 on six
@@ -542,7 +572,7 @@ inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspa
     constexpr double kFixupBytesPerSecond = 2e12;
     constexpr double kLaunchSeconds = 5e-6;
     constexpr int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
-    constexpr int kMostSplit = 8, kTailUnits = 2 * kCUs;
+    constexpr int kTailUnits = 2 * kCUs;
     X3Plan best{X3Shape::k128x256, 1, 0, 128, 256};
     double best_t = 1e300;
     for (const Option& o : options) {
@@ -565,7 +595,7 @@ inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspa
             for (const int split : kSplits) {
                 const int per = (blocks + split - 1) / split;
                 if (split > 1 && (per < 8 || (split - 1) * per >= blocks)) continue;
-                if (whole > 0 ? split == 1 || part * split > kTailUnits : split > kMostSplit) continue;
+                if (whole > 0 ? split == 1 || part * split > kTailUnits : split > o.most_split) continue;
                 const X3Plan plan{o.shape, split, t, o.bm, o.bn, whole};
                 if (plan.workspace_bytes() > workspace) continue;
                 double sec = (x3_estimate(whole, area, o.occupancy, o.rate) +
@@ -584,10 +614,6 @@ inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspa
         }
     }
     return best;
-}
-
-inline X3Shape x3_shape(int rows, int count, int cols, bool paired = false) {
-    return x3_plan(rows, count, cols, paired, 0).shape;
 }
 
 template <class P, class = void>
@@ -629,11 +655,17 @@ int launch_x3_tiles(P pol, int rows, int count, int cols, hipStream_t stream, in
 }
 
 // A launch by plan; `workspace` bytes at pol.part for split plans
-// (policies with a workspace; 0 otherwise).
-template <uint32_t QT, class P>
+// (policies with a workspace; 0 otherwise).  FEW: with the shapes for few A rows.
+template <uint32_t QT, bool FEW = false, class P>
 int launch_x3(const P& pol, int rows, int count, int cols, hipStream_t stream, size_t workspace = 0) {
-    const X3Plan plan = x3_plan(rows, count, cols, P::kPairedColumns, workspace);
+    const X3Plan plan = x3_plan(rows, count, cols, P::kPairedColumns, workspace, FEW);
     const int split = plan.split;
+    if constexpr (FEW) {
+        // 80 x 256 compute first, as the grouped MoE GEMMs run it.
+        if (plan.shape == X3Shape::k48x128) return launch_x3_tiles<QT, 1, 4, 3, 2, 1, false>(pol, rows, count, cols, stream, split);
+        if (plan.shape == X3Shape::k80x256) return launch_x3_tiles<QT, 1, 8, 5, 2, 1, true>(pol, rows, count, cols, stream, split);
+        if (plan.shape == X3Shape::k96x256) return launch_x3_tiles<QT, 2, 4, 3, 4, 1, false>(pol, rows, count, cols, stream, split, plan.whole);
+    }
     switch (plan.shape) {
         // The one-per-CU shapes with two stages of loads ahead: 1-3% faster
         // than one (and than compute-first) at 512-4096 tokens.

@@ -1249,15 +1249,15 @@ struct SharedDownAdd : TokenTiles {
 
 // part / part_bytes: the K split's workspace (none: no split).  Calls that
 // share it must be ordered, as calls on one stream are.
-template <uint32_t QT, class P>
+template <uint32_t QT, bool FEW = false, class P>
 int launch_token_gemm(P pol, int rows, hipStream_t stream, float* part = nullptr, size_t part_bytes = 0) {
     pol.part = part;
-    return launch_x3<QT>(pol, rows, pol.count, pol.cols, stream, part ? part_bytes : 0);
+    return launch_x3<QT, FEW>(pol, rows, pol.count, pol.cols, stream, part ? part_bytes : 0);
 }
 
 // Workspace bytes of the K split launch_x3 plans for a token GEMM.
-inline size_t token_gemm_part_bytes(int rows, int count, int cols, bool paired) {
-    return x3_plan(rows, count, cols, paired, static_cast<size_t>(-1)).workspace_bytes();
+inline size_t token_gemm_part_bytes(int rows, int count, int cols, bool paired, bool few = false) {
+    return x3_plan(rows, count, cols, paired, static_cast<size_t>(-1), few).workspace_bytes();
 }
 
 inline int launch_router_topk(const float* logits, int tokens, int experts, int top_k, int* ids, float* weights,
@@ -1555,7 +1555,7 @@ extern "C" int q3x_hip_moe_layer(const q3x_hip_moe_layer_weights* layer, const f
 }
 
 size_t q3x::gate_up_swiglu_workspace_bytes(int I, int H, int count) {
-    return I % 64 == 0 ? token_gemm_part_bytes(2 * I, count, H, true) : 0;
+    return I % 64 == 0 ? token_gemm_part_bytes(2 * I, count, H, true, true) : 0;
 }
 
 int q3x::gate_up_swiglu(const void* gate, const void* up, uint32_t type, int I, int H, const float* X, int count,
@@ -1574,8 +1574,8 @@ int q3x::gate_up_swiglu(const void* gate, const void* up, uint32_t type, int I, 
                                            : launch_thin<Q3X_HIP_MATRIX_Q4_0>(g, 2 * I, count, H, aligned16, stream);
     float* const part = aligned(workspace, 16) ? static_cast<float*>(workspace) : nullptr;
     return type == Q3X_HIP_MATRIX_Q8_0
-               ? launch_token_gemm<Q3X_HIP_MATRIX_Q8_0>(g, 2 * I, stream, part, workspace_bytes)
-               : launch_token_gemm<Q3X_HIP_MATRIX_Q4_0>(g, 2 * I, stream, part, workspace_bytes);
+               ? launch_token_gemm<Q3X_HIP_MATRIX_Q8_0, true>(g, 2 * I, stream, part, workspace_bytes)
+               : launch_token_gemm<Q3X_HIP_MATRIX_Q4_0, true>(g, 2 * I, stream, part, workspace_bytes);
 }
 
 int q3x::moe_layer_decode_add(const q3x_hip_moe_layer_weights& layer, const float* X, const uint16_t* norm_w,
