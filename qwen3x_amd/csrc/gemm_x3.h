@@ -477,10 +477,11 @@ __global__ __launch_bounds__(256) void gemm_x3_fixup_kernel(Policy pol, int rows
 // `few`.
 enum class X3Shape { k128x256, k64x128, k64x64, k128x192, k64x128_split, k48x128, k80x256, k96x256 };
 
-// A rows up to which x3_plan's `few` adds the shapes for few A rows: two 96-row
-// tiles.  Past it the other shapes' padding is small, and 193 to 256 rows gained
-// nothing.
-constexpr int kX3FewRows = 192;
+// A rows for which x3_plan's `few` adds the shapes for few A rows and takes the
+// rates measured there: up to two 96-row tiles.  Past them the other shapes'
+// padding is small, and 193 to 256 rows gained nothing; up to 32, gemm_thin.h
+// takes nearly every matrix.
+constexpr int kX3FewFrom = 33, kX3FewRows = 192;
 
 // Per-CU time of `tiles` tiles (or units) of `area` outputs each (in units
 // of area / (TFLOP/s): multiply by 2 K 256 / 1e12 for seconds).
@@ -519,17 +520,19 @@ struct X3Plan {
 // the partial-sum stores), and the launch adds the fixup: the units' sums
 // read back and the outputs written, and one more launch.
 //
-// few: with the shapes for few A rows (up to kX3FewRows).  A call of 77 rows
-// pays for 128 on the shapes above and one of 150 for 192 or 256; 80 x 256 and
-// 96 x 256 tiles hold them with 80 or 96 and 160 or 192 rows, 48 x 128 up to 48
-// (two of it lost to one 96 x 256).  Their K takes up to 16 splits: one A tile of
-// a 4096-row matrix is 16 to 32 tiles for 256 CUs.  The rates were fitted to a
+// few: with the shapes for few A rows (kX3FewFrom to kX3FewRows).  A call of 77
+// rows pays for 128 on the shapes above and one of 150 for 192 or 256; 80 x 256
+// and 96 x 256 tiles hold them with 80 or 96 and 160 or 192 rows, 48 x 128 up to
+// 48 (two of it lost to one 96 x 256).  K takes up to 16 splits there: one A
+// tile of a 4096-row matrix is 16 to 32 tiles for 256 CUs; and the 64 x 128
+// tiles on two K halves are taken over any K: with few tiles a CU has one, and
+// sixteen waves hide its loads better than eight.  The rates were fitted to a
 // sweep of every shape and split over 33 to 192 rows and 20 matrices (700 to
 // 20000 rows, 1024 to 24576 columns, Q8_0 and Q4_0); the plan's time there
-// against the one without these shapes, geometric means: 33-48 rows 0.89, 65-80
-// 0.84, 81-96 0.89, 129-160 0.87, 161-192 0.93, none slower by more than 3%
-// (49-64 and 97-128 rows keep the shapes above).  77 x 17408 x 5120 Q4_0 80.6
-// -> 65.0 us, 77 x 5120 x 17408 87.9 -> 61.5, 40 x 12288 x 4096 Q8_0 38.4 -> 32.7.
+// against the plan without all this: geometric mean 0.89, none slower by more
+// than 1%.  77 x 17408 x 5120 Q4_0 80.6 -> 65.0 us, 77 x 5120 x 17408 87.9 ->
+// 61.5, 40 x 12288 x 4096 Q8_0 38.4 -> 32.7, 128 x 5120 x 17408 Q4_0 (128 x 256
+// in 12 splits) about 92 -> 82.
 inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspace, bool few = false) {
     auto tiles = [&](int bm, int bn) {
         return static_cast<long long>((rows + bn - 1) / bn) * ((count + bm - 1) / bm);
@@ -540,27 +543,35 @@ inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspa
     static constexpr double r64[] = {150.0, 190.0, 215.0, 230.0};
     static constexpr double r192[] = {300.0};
     static constexpr double r64x128_split[] = {240.0};  // K halves on 16 waves, one workgroup per CU
-    static constexpr double r48[] = {132.0, 196.0, 180.0, 160.0};
-    static constexpr double r80[] = {267.0, 273.0};
-    static constexpr double r96[] = {300.0};
+    // Few A rows.
+    static constexpr double f256[] = {381.0};
+    static constexpr double f64x128[] = {204.0, 233.0, 260.0};
+    static constexpr double f64x128_long[] = {183.0, 240.0, 237.0};
+    static constexpr double f64[] = {146.0, 190.0, 170.0, 230.0};
+    static constexpr double f64x128_split[] = {222.0};
+    static constexpr double f48[] = {112.0, 188.0, 180.0, 160.0};
+    static constexpr double f80[] = {256.0, 273.0};
+    static constexpr double f96[] = {300.0};
     struct Option {
         X3Shape shape;
         int bm, bn, occupancy;
         const double* rate;
         bool ok;
-        int most_split = 8;
+        int most_split;
     };
     const bool long_k = cols >= kX3LongK;
-    few = few && count <= kX3FewRows;
+    few = few && count >= kX3FewFrom && count <= kX3FewRows;
+    const int most = few ? 16 : 8;
     const Option options[8] = {
-        {X3Shape::k128x256, 128, 256, 1, r256, true},
-        {X3Shape::k64x128, 64, 128, 3, long_k ? r64x128_long : r64x128, true},
-        {X3Shape::k64x64, 64, 64, 4, r64, true},
-        {X3Shape::k128x192, 128, 192, 1, r192, !paired},
-        {X3Shape::k64x128_split, 64, 128, 1, r64x128_split, long_k},
-        {X3Shape::k48x128, 48, 128, 4, r48, few && count <= 48, 16},
-        {X3Shape::k80x256, 80, 256, 2, r80, few, 16},
-        {X3Shape::k96x256, 96, 256, 1, r96, few, 16},
+        {X3Shape::k128x256, 128, 256, 1, few ? f256 : r256, true, most},
+        {X3Shape::k64x128, 64, 128, 3,
+         few ? (long_k ? f64x128_long : f64x128) : (long_k ? r64x128_long : r64x128), true, most},
+        {X3Shape::k64x64, 64, 64, 4, few ? f64 : r64, true, most},
+        {X3Shape::k128x192, 128, 192, 1, r192, !paired, most},
+        {X3Shape::k64x128_split, 64, 128, 1, few ? f64x128_split : r64x128_split, few || long_k, most},
+        {X3Shape::k48x128, 48, 128, 4, f48, few && count <= 48, most},
+        {X3Shape::k80x256, 80, 256, 2, f80, few, most},
+        {X3Shape::k96x256, 96, 256, 1, f96, few, 12},
     };
     const int blocks = cols / kBlock;
     // Fitted to a sweep of every shape at splits 1, 2, 3, 4, 6 and 8 on six

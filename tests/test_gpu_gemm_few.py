@@ -1,5 +1,5 @@
-"""GPU tests of the GEMM tiles for 33 to 192 tokens (48 x 128, 80 x 256 and 96
-x 256): token counts at and past each tile's edge, ragged rows and K ranges,
+"""GPU tests of the GEMM plans for 33 to 192 tokens (48 x 128, 80 x 256 and 96 x
+256 tiles, 64 x 128 on two K halves over short K, up to 16 splits): token counts at and past each tile's edge, ragged rows and K ranges,
 split over K and whole.  Against W x in float64 within the bound of the GEMM
 tests (1e-5 ||w|| ||x||), the split launch against the whole one, twice bit for
 bit, and accumulating; and the paired gate and up launch through an engine."""
@@ -13,14 +13,18 @@ from tests.test_gpu_parity import _torch, bits, dev, host, say
 
 pytestmark = pytest.mark.gpu
 
-TILES = {48: 128, 80: 256, 96: 256}
+TILES = {48: 128, 64: 128, 80: 256, 96: 256, 128: 256}
 
 
 # The tile height that each count is to take on these matrices.
+FEW = [(33, 48), (48, 48), (49, 64), (64, 64), (65, 80), (80, 80), (81, 96), (96, 96), (129, 80), (160, 80)]
+
+
 @pytest.mark.parametrize("type_", [Q8_0, Q4_0])
-@pytest.mark.parametrize("count,height", [(33, 48), (48, 48), (65, 80), (80, 80), (81, 96), (96, 96), (129, 80),
-                                          (160, 80), (161, 96), (192, 96)])
-@pytest.mark.parametrize("rows,cols", [(8300, 4128), (4097, 6144)])
+@pytest.mark.parametrize("rows,cols,count,height",
+                         [(rows, cols, *few) for rows, cols in [(8300, 4128), (4097, 6144)] for few in FEW] +
+                         [(4097, 6144, 97, 128), (4097, 6144, 128, 128), (4097, 6144, 161, 96), (4097, 6144, 192, 96),
+                          (8300, 4128, 161, 64), (8300, 4128, 192, 64)])
 def test_few_token_tiles(type_, rows, cols, count, height):
     torch = _torch()
     rng = np.random.default_rng(rows + cols + count + type_)
@@ -34,8 +38,8 @@ def test_few_token_tiles(type_, rows, cols, count, height):
     nbytes = q3x.gemm_workspace_bytes(lin, count)
     unit = -(-rows // TILES[height]) * -(-count // height) * height * TILES[height] * 4
     say(f"few-token tiles type={type_} {rows}x{cols} count={count} splits={nbytes / unit:g}")
-    assert nbytes > 0 and nbytes % unit == 0, "the plan must take this tile"
-    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda:0")
+    assert nbytes % unit == 0 and (nbytes > 0 or height == 64), "the plan must take this tile"
+    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device="cuda:0")
     Y, Y2 = (torch.full((count * rows + 8,), 3.0, dtype=torch.float32, device="cuda:0") for _ in range(2))
     q3x.batch_mv_ws(lin, Xd, Y, count, ws)
     got = host(Y)
@@ -67,7 +71,7 @@ def test_engine_prompts_against_single_tokens(type_):
         for i in range(len(tokens)):
             engine.forward(tokens[i:i + 1])
             want.append(engine.logits())
-        for prompt in (40, 77, 90, 160):
+        for prompt in (40, 64, 77, 90, 128, 160):
             say(f"engine type={type_}: prompt {prompt}")
             engine.reset()
             engine.forward(tokens[:prompt])
