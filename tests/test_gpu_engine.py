@@ -116,3 +116,20 @@ def test_checkpoint_reset_and_errors():
         e.forward(cont)
         assert e.position == 8
         assert np.array_equal(e.logits().view(np.uint32), after.view(np.uint32))
+
+
+def test_moe_prompt_shorter_than_the_chunk():
+    """A MoE layer's workspace does not grow with every token: 256 tokens of
+    this one ask for more than 257 do, and an engine for 257 takes them."""
+    _torch()
+    fields = dict(CONFIGS["moe_q4"], H=1024, I=512, shared_I=512, VH=8, KH=2, AH=4)
+    config, image, _ = synthetic_model(fields, seed=91)
+    weights = dev(image)
+    tokens = np.random.default_rng(91).integers(0, fields["V"], 256).astype(np.int32)
+    say("engine moe: prompt 256 in chunks of at most 257 and 512")
+    logits = []
+    for context in (257, 512):
+        with q3x.Engine(config, weights, context=context) as engine:
+            engine.forward(tokens)
+            logits.append(engine.logits())
+    assert np.all(np.abs(logits[0] - logits[1]) <= 2 * _bound(logits[1]))
