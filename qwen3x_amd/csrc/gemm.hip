@@ -82,13 +82,15 @@ int gemm(const void* w, uint32_t type, int rows, int cols, const float* X, int c
                                            : launch_thin<Q3X_HIP_MATRIX_Q4_0>(t, rows, count, cols, aligned(w, 16), stream);
     }
     // The split plan runs only with all of the workspace it asks for (16-byte
-    // aligned); otherwise q3x_hip_gemm's plan.
-    const size_t need = x3_plan(rows, count, cols, false, SIZE_MAX, true).workspace_bytes();
-    const size_t usable = need > 0 && aligned(workspace, 16) && workspace_bytes >= need ? need : 0;
+    // aligned); otherwise q3x_hip_gemm's plan.  A plan is about a microsecond
+    // of host work, so each is formed once.
+    const size_t usable = aligned(workspace, 16) ? workspace_bytes : 0;
+    X3Plan plan = x3_plan(rows, count, cols, false, usable ? SIZE_MAX : 0, true);
+    if (plan.workspace_bytes() > usable) plan = x3_plan(rows, count, cols, false, 0, true);
     DenseGemm g{0, X, cols, count, static_cast<const uint8_t*>(w), row_bytes, Y, rows, accumulate != 0, 0, 1,
                 static_cast<float*>(workspace)};
-    return type == Q3X_HIP_MATRIX_Q8_0 ? launch_x3<Q3X_HIP_MATRIX_Q8_0, true>(g, rows, count, cols, stream, usable)
-                                       : launch_x3<Q3X_HIP_MATRIX_Q4_0, true>(g, rows, count, cols, stream, usable);
+    return type == Q3X_HIP_MATRIX_Q8_0 ? launch_x3_plan<Q3X_HIP_MATRIX_Q8_0, true>(g, plan, rows, count, cols, stream)
+                                       : launch_x3_plan<Q3X_HIP_MATRIX_Q4_0, true>(g, plan, rows, count, cols, stream);
 }
 
 }  // namespace

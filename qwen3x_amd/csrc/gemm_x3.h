@@ -665,11 +665,11 @@ int launch_x3_tiles(P pol, int rows, int count, int cols, hipStream_t stream, in
     return launch_status();
 }
 
-// A launch by plan; `workspace` bytes at pol.part for split plans
-// (policies with a workspace; 0 otherwise).  FEW: with the shapes for few A rows.
+// The launch of `plan` (x3_plan's, for these sizes and the policy's
+// kPairedColumns; split plans need pol.part).  FEW: with the shapes for few A
+// rows.
 template <uint32_t QT, bool FEW = false, class P>
-int launch_x3(const P& pol, int rows, int count, int cols, hipStream_t stream, size_t workspace = 0) {
-    const X3Plan plan = x3_plan(rows, count, cols, P::kPairedColumns, workspace, FEW);
+int launch_x3_plan(const P& pol, const X3Plan& plan, int rows, int count, int cols, hipStream_t stream) {
     const int split = plan.split;
     if constexpr (FEW) {
         // 80 x 256 compute first, as the grouped MoE GEMMs run it.
@@ -695,6 +695,14 @@ int launch_x3(const P& pol, int rows, int count, int cols, hipStream_t stream, s
             return launch_x3_tiles<QT, 2, 4, 2, 2, 1, false>(pol, rows, count, cols, stream, split);
         default: return launch_x3_tiles<QT, 2, 2, 2, 2, 1, false>(pol, rows, count, cols, stream, split);
     }
+}
+
+// The launch of the best plan that fits `workspace` bytes at pol.part
+// (policies with a workspace; 0 otherwise).
+template <uint32_t QT, bool FEW = false, class P>
+int launch_x3(const P& pol, int rows, int count, int cols, hipStream_t stream, size_t workspace = 0) {
+    return launch_x3_plan<QT, FEW>(pol, x3_plan(rows, count, cols, P::kPairedColumns, workspace, FEW), rows, count, cols,
+                                   stream);
 }
 
 }  // namespace q3x
