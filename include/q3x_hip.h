@@ -99,19 +99,22 @@ int q3x_hip_gemm(const void* w, uint32_t type, int rows, int cols,
                  hipStream_t stream);
 
 /* Bytes of caller-owned workspace with which q3x_hip_gemm_ws splits the K
- * dimension of this GEMM over workgroups (0: it would not split).  For the
- * same shape and arguments as q3x_hip_gemm, with a workspace of at least
- * q3x_hip_gemm_workspace_bytes(type, rows, cols, count) bytes (16-byte
- * aligned; smaller or null runs q3x_hip_gemm's launch): a launch of few
+ * dimension of this GEMM over workgroups (0: it would not split), enough for
+ * every smaller count of the same matrix too: a caller may size one workspace
+ * for its most tokens.  For the same shape and arguments as q3x_hip_gemm, with
+ * a workspace of at least that size (16-byte aligned; one too small for the
+ * count's partial sums, or null, runs q3x_hip_gemm's launch): a launch of few
  * output tiles over a long K (e.g. 512 tokens x 5120 rows x 17408 columns),
  * or the last, short round of one of a few more tiles than the chip runs at
- * once (512 x 17408 x 5120), then fills the chip, each tile's K ranges summed by a second launch in K
- * order.  Deterministic; the sums run in another order than q3x_hip_gemm's,
- * within the same tolerance against the reference.  The workspace holds the
- * partial sums from the first launch to the second, so calls that share one
- * must be ordered (e.g. issued on one stream).  Same role as
- * q3x_hip_gemm (batch_mv, arch/cuda/engine.cu:1568); no counterpart of its
- * own in the reference. */
+ * once (512 x 17408 x 5120), then fills the chip, each tile's K ranges summed
+ * by a second launch in K order.  Deterministic; the sums run in another order
+ * than q3x_hip_gemm's, within the same tolerance against the reference.  Up to
+ * 32 tokens the workspace is used only where w is not 4-byte aligned, or by 17
+ * tokens or more on rows past 16384 columns; the other calls read the weights
+ * once without one.  The workspace holds the partial sums from the first
+ * launch to the second, so calls that share one must be ordered (e.g. issued
+ * on one stream).  Same role as q3x_hip_gemm (batch_mv,
+ * arch/cuda/engine.cu:1568); no counterpart of its own in the reference. */
 size_t q3x_hip_gemm_workspace_bytes(uint32_t type, int rows, int cols, int count);
 int q3x_hip_gemm_ws(const void* w, uint32_t type, int rows, int cols,
                     const float* X, int count, float* Y, int accumulate,

@@ -277,13 +277,14 @@ def batch_mv(linear: Linear, X, Y, count: int, add: bool = False, stream=None):
 
 def gemm_workspace_bytes(linear: Linear, count: int) -> int:
     """Bytes of workspace with which batch_mv_ws splits K over workgroups
-    for `count` tokens (0: no split)."""
+    for `count` tokens (0: no split); enough for every smaller count too."""
     return int(lib().q3x_hip_gemm_workspace_bytes(linear.type, linear.rows, linear.columns, count))
 
 
 def batch_mv_ws(linear: Linear, X, Y, count: int, workspace, add: bool = False, stream=None):
     """batch_mv with a workspace (a device tensor of at least
-    gemm_workspace_bytes(linear, count) bytes, or None)."""
+    gemm_workspace_bytes(linear, count) bytes, this count's or a larger one's,
+    or None)."""
     _need_device(linear.weight, X, Y)
     ws, nbytes = (0, 0) if workspace is None else (_ptr(workspace), workspace.numel() * workspace.element_size())
     if workspace is not None:

@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "common.h"
+#include "gemm.h"
 #include "matvec.h"
 #include "moe.h"
 #include "rows.h"
@@ -2021,7 +2022,7 @@ extern "C" int q3x_hip_engine_create(const q3x_hip_model_config* config, const v
             if (!m.w || !asked.emplace(m.rows, m.cols).second) return most;
             for (size_t n = 16; n < R + 16; n += 16) {
                 const int count = static_cast<int>(std::min(n, R));
-                most = std::max(most, q3x_hip_gemm_workspace_bytes(c.matrix_type, m.rows, m.cols, count));
+                most = std::max(most, gemm_split_bytes(m.rows, m.cols, count));
             }
             return most;
         };

@@ -18,6 +18,10 @@ namespace q3x {
 
 constexpr int kXcds = 8;  // MI355X: 8 XCDs of 32 CUs
 
+// Bytes of the K split that q3x_hip_gemm_ws runs for this count of tokens (0:
+// none); q3x_hip_gemm_workspace_bytes asks for the smaller counts' too.
+size_t gemm_split_bytes(int rows, int cols, int count);
+
 struct GemmTile {
     int m0;      // first A row of the tile (policy-defined numbering)
     int mcount;  // valid A rows in the tile (<= BM)

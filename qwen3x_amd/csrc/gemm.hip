@@ -6,6 +6,9 @@
 // path is an FP32 SIMT kernel (batch_mv_q8_kernel :761, 64 rows x 128 tokens
 // per CTA) and which has no Q4_0 GEMM (it asserts, :1580).
 #include "gemm.h"
+
+#include <algorithm>
+
 #include "gemm_thin.h"
 #include "gemm_x3.h"
 #include "matvec.h"
@@ -93,7 +96,33 @@ int gemm(const void* w, uint32_t type, int rows, int cols, const float* X, int c
                                        : launch_x3_plan<Q3X_HIP_MATRIX_Q4_0, true>(g, plan, rows, count, cols, stream);
 }
 
+// What q3x_hip_gemm_workspace_bytes asks for: the bytes of this count's plan,
+// or more where a smaller count's plan needs more, in whole copies of this
+// plan's tiles.  Plans do not grow with the count (12288 x 4096: 18 MiB at 96
+// tokens, 8 at 192, whose plan splits a few tiles only), and a split plan
+// runs with all of its bytes or not at all, so a workspace sized once for a
+// caller's most tokens has to hold the smaller counts' too: with the plan's
+// own bytes alone, 128 tokens x 4096 x 12288 with the workspace of 192 ran
+// unsplit in 222 us, 96 x 12288 x 4096 in 70; with them 54 and 48 (Q4_0 and
+// Q8_0).  Plans change where a tile's height divides the count: at multiples
+// of 16 up to kX3FewRows, of 64 past it, where a count that would not split
+// asks for nothing.
+size_t gemm_request(int rows, int cols, int count) {
+    const X3Plan plan = x3_plan(rows, count, cols, false, SIZE_MAX, true);
+    const size_t own = plan.workspace_bytes();
+    if (own == 0 && count > kX3FewRows) return 0;
+    size_t most = own;
+    for (int n = 16; n < count; n += n < kX3FewRows ? 16 : 64)
+        most = std::max(most, gemm_split_bytes(rows, cols, n));
+    const size_t copy = static_cast<size_t>(plan.tiles - plan.whole) * plan.bm * plan.bn * 4;
+    return (most + copy - 1) / copy * copy;
+}
+
 }  // namespace
+
+size_t q3x::gemm_split_bytes(int rows, int cols, int count) {
+    return x3_plan(rows, count, cols, false, SIZE_MAX, true).workspace_bytes();
+}
 
 extern "C" int q3x_hip_gemm(const void* w, uint32_t type, int rows, int cols, const float* X,
                             int count, float* Y, int accumulate, hipStream_t stream) {
@@ -103,7 +132,7 @@ extern "C" int q3x_hip_gemm(const void* w, uint32_t type, int rows, int cols, co
 extern "C" size_t q3x_hip_gemm_workspace_bytes(uint32_t type, int rows, int cols, int count) {
     size_t bytes;
     if (type == Q3X_HIP_MATRIX_BF16 || count <= 0 || !quantized_size(type, rows, cols, &bytes)) return 0;
-    return x3_plan(rows, count, cols, false, SIZE_MAX, true).workspace_bytes();
+    return gemm_request(rows, cols, count);
 }
 
 extern "C" int q3x_hip_gemm_ws(const void* w, uint32_t type, int rows, int cols, const float* X, int count,

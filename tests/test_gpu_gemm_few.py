@@ -57,6 +57,28 @@ def test_few_token_tiles(type_, rows, cols, count, height):
 
 
 @pytest.mark.parametrize("type_", [Q8_0, Q4_0])
+@pytest.mark.parametrize("rows,cols,most,counts", [(12288, 4096, 192, (40, 64, 80, 96, 128)), (4096, 12288, 192, (96, 128)),
+                                                   (17408, 5120, 512, (176, 256))])
+def test_workspace_sized_for_more_tokens(type_, rows, cols, most, counts):
+    """The workspace of a larger count keeps the split: the bits of a call with
+    the count's own, and not those of the unsplit launch."""
+    torch = _torch()
+    rng = np.random.default_rng(rows + type_)
+    lin = q3x.Linear(dev(random_blocks(rng, type_, rows, cols)), rows, cols, type_)
+    shared = torch.empty(q3x.gemm_workspace_bytes(lin, most), dtype=torch.uint8, device="cuda:0")
+    for count in counts:
+        say(f"workspace of {most} tokens type={type_} {rows}x{cols} count={count}")
+        X = dev(rng.normal(0, 1, (count, cols)).astype(np.float32))
+        own = torch.empty(q3x.gemm_workspace_bytes(lin, count), dtype=torch.uint8, device="cuda:0")
+        Y = [torch.full((count, rows), 3.0, dtype=torch.float32, device="cuda:0") for _ in range(3)]
+        q3x.batch_mv_ws(lin, X, Y[0], count, shared)
+        q3x.batch_mv_ws(lin, X, Y[1], count, own)
+        q3x.batch_mv(lin, X, Y[2], count)
+        assert torch.equal(Y[0].view(torch.int32), Y[1].view(torch.int32))
+        assert not torch.equal(Y[0].view(torch.int32), Y[2].view(torch.int32))
+
+
+@pytest.mark.parametrize("type_", [Q8_0, Q4_0])
 def test_engine_prompts_against_single_tokens(type_):
     """Prompts' GEMMs (the paired gate and up launch among them) against the
     same tokens one by one, each within the engine tests' bound of the

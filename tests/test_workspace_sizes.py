@@ -1,0 +1,31 @@
+"""Workspace sizes on the host: a workspace sized once for a caller's most
+tokens serves every smaller count of the same matrix or layer."""
+import ctypes
+
+import pytest
+
+import qwen3x_amd as q3x
+from tests.helpers import Q4_0, Q8_0
+
+
+def _split_bytes(rows, cols, count):
+    """Bytes of the partial sums that the call itself writes (q3x::gemm_split_bytes)."""
+    f = q3x.lib()["_ZN3q3x16gemm_split_bytesEiii"]
+    f.restype, f.argtypes = ctypes.c_size_t, [ctypes.c_int] * 3
+    return f(rows, cols, count)
+
+
+@pytest.mark.parametrize("rows,cols", [(12288, 4096), (4096, 12288), (5120, 17408), (1024, 5120), (6144, 2048),
+                                       (24576, 5120), (700, 3072), (8300, 4128), (40000, 1024)])
+def test_gemm_workspace_holds_smaller_counts(rows, cols):
+    size = q3x.lib().q3x_hip_gemm_workspace_bytes
+    most = [0]
+    for count in range(1, 1301):
+        most.append(max(most[-1], _split_bytes(rows, cols, count)))
+    for count in list(range(2, 200, 3)) + [192, 193, 255, 256, 257, 511, 512, 640, 1300]:
+        nbytes = size(Q8_0, rows, cols, count)
+        assert nbytes == size(Q4_0, rows, cols, count)
+        if count <= 192 or _split_bytes(rows, cols, count):
+            assert nbytes >= most[count], count
+        else:
+            assert nbytes == 0, count
