@@ -472,9 +472,11 @@ __global__ __launch_bounds__(256) void gemm_x3_fixup_kernel(Policy pol, int rows
 // x 12288 (64 tiles of 128 x 256) 208 on 64 x 128.
 //
 // 48 x 128 (4 waves of 48x32, four workgroups per CU), 80 x 256 (8 waves of
-// 80x32, two) and 96 x 256 (8 waves of 48x64, one) are for few A rows, where
+// 80x32) and 96 x 256 (8 waves of 48x64, both one) are for few A rows, where
 // the rows a tile is padded by are work done for nothing: see x3_plan's
-// `few`.
+// `few`.  (80 x 256 takes 140 registers for Q4_0 and 144 for Q8_0 with the
+// policies that use it here, three waves a SIMD; with the grouped MoE GEMMs'
+// policies it takes 124 and 128, and two workgroups share a CU.)
 enum class X3Shape { k128x256, k64x128, k64x64, k128x192, k64x128_split, k48x128, k80x256, k96x256 };
 
 // A rows for which x3_plan's `few` adds the shapes for few A rows and takes the
@@ -526,13 +528,17 @@ struct X3Plan {
 // 48 (two of it lost to one 96 x 256).  K takes up to 16 splits there: one A
 // tile of a 4096-row matrix is 16 to 32 tiles for 256 CUs; and the 64 x 128
 // tiles on two K halves are taken over any K: with few tiles a CU has one, and
-// sixteen waves hide its loads better than eight.  The rates were fitted to a
-// sweep of every shape and split over 33 to 192 rows and 20 matrices (700 to
-// 20000 rows, 1024 to 24576 columns, Q8_0 and Q4_0); the plan's time there
-// against the plan without all this: geometric mean 0.89, none slower by more
-// than 1%.  77 x 17408 x 5120 Q4_0 80.6 -> 65.0 us, 77 x 5120 x 17408 87.9 ->
-// 61.5, 40 x 12288 x 4096 Q8_0 38.4 -> 32.7, 128 x 5120 x 17408 Q4_0 (128 x 256
-// in 12 splits) about 92 -> 82.
+// sixteen waves hide its loads better than eight.  Its halves fill and drain a
+// pipeline each over half the blocks, so it pays for a round unsplit too.  The
+// rates and costs were fitted to a sweep of every shape, split and tail over
+// 40 to 192 rows and 24 matrices (700 to 40000 rows, 1024 to 24576 columns),
+// Q8_0 and Q4_0, with a workspace and without; the chosen plan's time there
+// against that of the plan without all this (geometric mean, worst): with a
+// workspace Q8_0 0.87, 1.05 (128 x 1024 x 4096, 18.0 -> 18.9 us) and Q4_0 0.90,
+// 1.02; without 0.87, 1.03 and 0.83, 1.00; over 26 other matrices 0.88, 1.05
+// and 0.83, none slower.  77 x 17408 x 5120
+// Q4_0 80.6 -> 65.0 us, 77 x 5120 x 17408 87.9 -> 61.5, 40 x 12288 x 4096 Q8_0
+// 38.4 -> 32.7, 128 x 5120 x 17408 Q4_0 (128 x 256 in 12 splits) about 92 -> 82.
 inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspace, bool few = false) {
     auto tiles = [&](int bm, int bn) {
         return static_cast<long long>((rows + bn - 1) / bn) * ((count + bm - 1) / bm);
@@ -544,14 +550,15 @@ inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspa
     static constexpr double r192[] = {300.0};
     static constexpr double r64x128_split[] = {240.0};  // K halves on 16 waves, one workgroup per CU
     // Few A rows.
-    static constexpr double f256[] = {381.0};
-    static constexpr double f64x128[] = {204.0, 233.0, 260.0};
-    static constexpr double f64x128_long[] = {183.0, 240.0, 237.0};
-    static constexpr double f64[] = {146.0, 190.0, 170.0, 230.0};
+    static constexpr double f256[] = {337.0};
+    static constexpr double f64x128[] = {192.0, 226.0, 254.0};
+    static constexpr double f64x128_long[] = {192.0, 227.0, 238.0};
+    static constexpr double f64[] = {101.0, 172.0, 184.0, 196.0};
+    static constexpr double f192[] = {276.0};
     static constexpr double f64x128_split[] = {222.0};
-    static constexpr double f48[] = {112.0, 188.0, 180.0, 160.0};
-    static constexpr double f80[] = {256.0, 273.0};
-    static constexpr double f96[] = {300.0};
+    static constexpr double f48[] = {107.0, 187.0, 202.0, 144.0};
+    static constexpr double f80[] = {258.0};
+    static constexpr double f96[] = {272.0};
     struct Option {
         X3Shape shape;
         int bm, bn, occupancy;
@@ -567,10 +574,10 @@ inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspa
         {X3Shape::k64x128, 64, 128, 3,
          few ? (long_k ? f64x128_long : f64x128) : (long_k ? r64x128_long : r64x128), true, most},
         {X3Shape::k64x64, 64, 64, 4, few ? f64 : r64, true, most},
-        {X3Shape::k128x192, 128, 192, 1, r192, !paired, most},
+        {X3Shape::k128x192, 128, 192, 1, few ? f192 : r192, !paired, most},
         {X3Shape::k64x128_split, 64, 128, 1, few ? f64x128_split : r64x128_split, few || long_k, most},
         {X3Shape::k48x128, 48, 128, 4, f48, few && count <= 48, most},
-        {X3Shape::k80x256, 80, 256, 2, f80, few, most},
+        {X3Shape::k80x256, 80, 256, 1, f80, few, most},
         {X3Shape::k96x256, 96, 256, 1, f96, few, 12},
     };
     const int blocks = cols / kBlock;
@@ -579,8 +586,8 @@ inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspa
     // choice is within 2% of the fastest on each.  A unit's pipeline fill and
     // drain cost per round (less where other resident units hide them), and
     // the fixup's traffic moves at about a quarter of HBM's peak.
-    constexpr double kRoundSeconds = 3e-6, kRoundSecondsShared = 2e-6;
-    constexpr double kFixupBytesPerSecond = 2e12;
+    const double round = few ? 2.5e-6 : 3e-6, round_shared = few ? 2.6e-6 : 2e-6;
+    const double fixup_rate = few ? 2.4e12 : 2e12;
     constexpr double kLaunchSeconds = 5e-6;
     constexpr int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
     constexpr int kTailUnits = 2 * kCUs;
@@ -605,7 +612,7 @@ inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspa
             const long long part = t - whole;
             for (const int split : kSplits) {
                 const int per = (blocks + split - 1) / split;
-                if (split > 1 && (per < 8 || (split - 1) * per >= blocks)) continue;
+                if (split > 1 && (per < (o.shape == X3Shape::k64x128_split ? 16 : 8) || (split - 1) * per >= blocks)) continue;
                 if (whole > 0 ? split == 1 || part * split > kTailUnits : split > o.most_split) continue;
                 const X3Plan plan{o.shape, split, t, o.bm, o.bn, whole};
                 if (plan.workspace_bytes() > workspace) continue;
@@ -614,9 +621,11 @@ inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspa
                 if (split > 1) {
                     const long long more = (part * split + static_cast<long long>(kCUs) * o.occupancy - 1) /
                                            (static_cast<long long>(kCUs) * o.occupancy);
-                    sec += more * (o.occupancy == 1 ? kRoundSeconds : kRoundSecondsShared) + kLaunchSeconds +
-                           static_cast<double>(part) * area * 4.0 * (split + 1) / kFixupBytesPerSecond;
+                    sec += more * (o.occupancy == 1 ? round : round_shared) + kLaunchSeconds +
+                           static_cast<double>(part) * area * 4.0 * (split + 1) / fixup_rate;
                 }
+                if (few && o.shape == X3Shape::k64x128_split)
+                    sec += ((split > 1 ? whole : t) + kCUs - 1) / kCUs * round;
                 if (sec < best_t) {
                     best_t = sec;
                     best = plan;
@@ -674,7 +683,7 @@ int launch_x3_plan(const P& pol, const X3Plan& plan, int rows, int count, int co
     if constexpr (FEW) {
         // 80 x 256 compute first, as the grouped MoE GEMMs run it.
         if (plan.shape == X3Shape::k48x128) return launch_x3_tiles<QT, 1, 4, 3, 2, 1, false>(pol, rows, count, cols, stream, split);
-        if (plan.shape == X3Shape::k80x256) return launch_x3_tiles<QT, 1, 8, 5, 2, 1, true>(pol, rows, count, cols, stream, split);
+        if (plan.shape == X3Shape::k80x256) return launch_x3_tiles<QT, 1, 8, 5, 2, 1, true>(pol, rows, count, cols, stream, split, plan.whole);
         if (plan.shape == X3Shape::k96x256) return launch_x3_tiles<QT, 2, 4, 3, 4, 1, false>(pol, rows, count, cols, stream, split, plan.whole);
     }
     switch (plan.shape) {
