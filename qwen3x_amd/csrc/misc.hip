@@ -124,9 +124,11 @@ __device__ __forceinline__ void load_eight(const uint16_t* __restrict__ src, siz
 // lanes of a quad share a block, eight values each, so a wave reads 1 KB (BF16)
 // contiguous per load; the block's maximum and, for Q4_0, the other half's
 // nibbles are exchanged by DPP inside the quad.  A workgroup packs
-// kQuantBlocks blocks into LDS and writes them out as one contiguous run,
-// 16 bytes a lane where dst is 16-byte aligned (kQuantBlocks blocks are a
-// multiple of 16 bytes in either format), single bytes otherwise.  One thread
+// kQuantBlocks blocks into LDS and writes them out as one contiguous run of
+// 16-byte words (kQuantBlocks blocks are a multiple of 16 bytes in either
+// format); where dst is not 16-byte aligned, the words inside the run, put
+// together from LDS dwords, and single bytes around them (all in single bytes
+// 5001 x 2080 BF16 values to Q8_0 took 9.5 us, 8.6 so).  One thread
 // per block, with 64- or 128-byte strided loads and 18 or 34 byte stores of
 // its own, took 140 us for 17408 x 5120 BF16 values (1.6 TB/s); the figures of
 // this form are beside dequant_kernel.
@@ -141,7 +143,7 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_kernel(const Src* __re
     constexpr int BB = QT == Q3X_HIP_MATRIX_Q8_0 ? kQ8Bytes : kQ4Bytes;
     constexpr int kRounds = kQuantBlocks * 4 / kQuantThreads;
     static_assert(kQuantBlocks * BB % 16 == 0, "a workgroup's run is whole 16-byte words");
-    __shared__ __attribute__((aligned(16))) uint8_t packed[kQuantBlocks * BB];
+    __shared__ __attribute__((aligned(16))) uint8_t packed[kQuantBlocks * BB + 16];  // and a dword past the last word
     const size_t block0 = static_cast<size_t>(blockIdx.x) * kQuantBlocks;
     const int part = threadIdx.x & 3;  // eighth values 8 * part .. + 7 of the block
     float v[kRounds][8];
@@ -223,10 +225,26 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_kernel(const Src* __re
     __syncthreads();
     const int bytes = static_cast<int>(min(static_cast<size_t>(kQuantBlocks), blocks - block0)) * BB;
     uint8_t* run = dst + block0 * BB;
-    const int words = wide ? bytes / 16 : 0;
-    for (int i = threadIdx.x; i < words; i += kQuantThreads)
-        reinterpret_cast<u32x4*>(run)[i] = reinterpret_cast<const u32x4*>(packed)[i];
-    for (int i = 16 * words + threadIdx.x; i < bytes; i += kQuantThreads) run[i] = packed[i];
+    // Bytes before the first 16-byte boundary of dst, and words after them.
+    const int head = wide ? 0 : min(bytes, static_cast<int>(-reinterpret_cast<uintptr_t>(run) & 15));
+    const int words = (bytes - head) / 16;
+    if (wide) {
+        for (int i = threadIdx.x; i < words; i += kQuantThreads)
+            reinterpret_cast<u32x4*>(run)[i] = reinterpret_cast<const u32x4*>(packed)[i];
+    } else {
+        const uint32_t* dwords = reinterpret_cast<const uint32_t*>(packed) + head / 4;
+        for (int i = threadIdx.x; i < words; i += kQuantThreads) {
+            uint32_t w[5];
+#pragma unroll
+            for (int j = 0; j < 5; ++j) w[j] = dwords[4 * i + j];
+            u32x4 v;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = __builtin_amdgcn_alignbyte(w[j + 1], w[j], head & 3);
+            reinterpret_cast<u32x4*>(run + head)[i] = v;
+        }
+        if (threadIdx.x < head) run[threadIdx.x] = packed[threadIdx.x];
+    }
+    for (int i = head + 16 * words + threadIdx.x; i < bytes; i += kQuantThreads) run[i] = packed[i];
 }
 
 }  // namespace q3x

@@ -58,3 +58,21 @@ def test_dequant_run_edges(type_, offset, rows, cols):
     got = host(out)
     assert np.array_equal(got[offset:offset + rows * cols].reshape(rows, cols).view(np.uint32), want.view(np.uint32))
     assert np.all(got[:offset] == -7.0) and np.all(got[offset + rows * cols:] == -7.0)
+
+
+@pytest.mark.parametrize("type_", [Q8_0, Q4_0])
+@pytest.mark.parametrize("blocks", [1, 257])
+def test_quantize_every_alignment(type_, blocks):
+    """Destinations at every byte of a 16-byte word, a run shorter than one
+    and runs of whole words between single bytes."""
+    torch = _torch()
+    v = _values(blocks)
+    want = oracle.quantize(type_, v)
+    src = dev(v)
+    say(f"quantize type={type_} blocks={blocks} at offsets 0 to 16")
+    for offset in range(17):
+        buf = torch.full((offset + want.size + 16,), 0xA5, dtype=torch.uint8, device="cuda:0")
+        q3x.quantize(type_, src, blocks, 32, buf[offset:])
+        got = host(buf)
+        assert np.array_equal(got[offset:offset + want.size], want)
+        assert np.all(got[:offset] == 0xA5) and np.all(got[offset + want.size:] == 0xA5)
