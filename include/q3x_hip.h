@@ -138,7 +138,8 @@ int q3x_hip_dequant(const void* w, uint32_t type, int cols, int row0, int nrows,
 int q3x_hip_router_topk(const float* logits, int tokens, int experts, int top_k,
                         int* ids, float* weights, hipStream_t stream);
 
-/* Bytes of caller-owned workspace q3x_hip_moe_routed needs. */
+/* Bytes of caller-owned workspace q3x_hip_moe_routed needs; fewer tokens need
+ * no more. */
 size_t q3x_hip_moe_workspace_bytes(int tokens, int experts, int top_k, int H, int I);
 
 /* Routed experts: for every token t,

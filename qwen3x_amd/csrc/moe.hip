@@ -308,7 +308,6 @@ struct MoeLayout {
     size_t chunk_counts;
     int chunks;
     size_t gu, h, d, total;
-    int max_tiles;
     int thin;  // tile height of the few-pair grouped GEMMs; 0: the 80-pair tiles
 };
 
@@ -333,24 +332,37 @@ inline int moe_thin_height(int tokens, int experts, int top_k) {
     return mean <= 2.0 ? 4 : mean <= 5.0 ? 8 : mean <= 11.0 ? 16 : mean <= 24.0 && live <= 16.0 ? 32 : 0;
 }
 
-inline MoeLayout moe_layout(int tokens, int experts, int top_k, int H, int I, int thin) {
+// The most tiles of bm pairs that `pairs` pairs of `experts` experts fill.
+inline int moe_tiles(size_t pairs, int experts, int bm) {
+    return static_cast<int>(pairs / bm + std::min<size_t>(experts, pairs) + 1);
+}
+
+// Entries of the tile table: enough for every tile height, and no fewer than
+// fewer tokens have, so that a workspace sized for a caller's most tokens
+// holds every smaller call.  Few-pair tiles take a token count of at most 2, 5
+// or 11 pairs an expert in tiles of 4, 8 or 16, so at most 11 / 16 of a tile an
+// expert past the first, and at most 24 pairs of at most 16 experts in tiles
+// of 32.
+inline int moe_table_entries(size_t pairs, int experts) {
+    const size_t few = std::min<size_t>(pairs / 4, std::max<size_t>(static_cast<size_t>(experts) * 11 / 16, 12));
+    return moe_tiles(pairs, experts, kGrpBM) + static_cast<int>(few > pairs / kGrpBM ? few - pairs / kGrpBM : 0);
+}
+
+inline MoeLayout moe_layout(int tokens, int experts, int top_k, int H, int I, int table) {
     MoeLayout L{};
     const size_t P = static_cast<size_t>(tokens) * top_k;
     size_t off = 0;
     auto take = [&](size_t bytes) { const size_t at = off; off = align_up(off + bytes, 256); return at; };
-    {  // grouping arrays (also for one token: the fallback of unaligned decode shapes)
-        L.thin = thin;
-        L.max_tiles = static_cast<int>(P / (thin ? thin : kGrpBM) + std::min<size_t>(experts, P) + 1);
-        L.ntiles = take(sizeof(int));
-        L.nvalid = take(sizeof(int));
-        L.tile_expert = take(sizeof(int) * L.max_tiles);
-        L.tile_start = take(sizeof(int) * L.max_tiles);
-        L.tile_count = take(sizeof(int) * L.max_tiles);
-        L.pos_of_pair = take(sizeof(int) * P);
-        L.src_token = take(sizeof(int) * P);
-        L.chunks = static_cast<int>((P + kChunk - 1) / kChunk);
-        L.chunk_counts = take(sizeof(int) * static_cast<size_t>(L.chunks) * experts);
-    }
+    // Grouping arrays (also for one token: the fallback of unaligned decode shapes).
+    L.ntiles = take(sizeof(int));
+    L.nvalid = take(sizeof(int));
+    L.tile_expert = take(sizeof(int) * table);
+    L.tile_start = take(sizeof(int) * table);
+    L.tile_count = take(sizeof(int) * table);
+    L.pos_of_pair = take(sizeof(int) * P);
+    L.src_token = take(sizeof(int) * P);
+    L.chunks = static_cast<int>((P + kChunk - 1) / kChunk);
+    L.chunk_counts = take(sizeof(int) * static_cast<size_t>(L.chunks) * experts);
     L.gu = take(sizeof(float) * P * 2 * I);
     L.h = take(sizeof(float) * P * I);
     L.d = take(sizeof(float) * P * H);
@@ -359,15 +371,23 @@ inline MoeLayout moe_layout(int tokens, int experts, int top_k, int H, int I, in
 }
 
 inline MoeLayout moe_layout(int tokens, int experts, int top_k, int H, int I) {
-    const MoeLayout wide = moe_layout(tokens, experts, top_k, H, I, 0);
-    const int thin = tokens > 1 ? moe_thin_height(tokens, experts, top_k) : 0;
-    if (thin == 0) return wide;
-    const MoeLayout L = moe_layout(tokens, experts, top_k, H, I, thin);
-    // More tiles than a grid holds stay on the wide ones.
-    if (static_cast<long long>(L.max_tiles) * (std::max(2LL * I, static_cast<long long>(H)) / 32 + 1) > (1 << 22)) return wide;
-    // The longer tile table must not push a request past the static scratch
-    // that held it.
-    if (L.total > Q3X_HIP_NOALLOC_SCRATCH_BYTES && wide.total <= Q3X_HIP_NOALLOC_SCRATCH_BYTES) return wide;
+    const size_t P = static_cast<size_t>(tokens) * top_k;
+    MoeLayout L = moe_layout(tokens, experts, top_k, H, I, moe_table_entries(P, experts));
+    if (L.total > Q3X_HIP_NOALLOC_SCRATCH_BYTES) {
+        // The longer tile table must not push a request past the static
+        // scratch that holds it with the 80-pair tiles' table: it asks for
+        // all of the scratch (no less than fewer tokens ask for).
+        MoeLayout wide = moe_layout(tokens, experts, top_k, H, I, moe_tiles(P, experts, kGrpBM));
+        if (wide.total <= Q3X_HIP_NOALLOC_SCRATCH_BYTES) {
+            wide.total = Q3X_HIP_NOALLOC_SCRATCH_BYTES;
+            return wide;
+        }
+    }
+    L.thin = tokens > 1 ? moe_thin_height(tokens, experts, top_k) : 0;
+    // More tiles than a grid holds stay on the 80-pair ones.
+    if (L.thin && static_cast<long long>(moe_tiles(P, experts, L.thin)) *
+                          (std::max(2LL * I, static_cast<long long>(H)) / 32 + 1) > (1 << 22))
+        L.thin = 0;
     return L;
 }
 
@@ -1035,7 +1055,7 @@ int moe_grouped(const uint8_t* gate_up, const uint8_t* down, int experts, int H,
     }
     if ((status = launch_status()) != Q3X_HIP_OK) return status;
 
-    const int tiles_bound = L.max_tiles;
+    const int tiles_bound = moe_tiles(P, experts, bm);
     const double tiles = moe_live_experts(tokens, experts, top_k);  // live tiles, about
     if (I % 64 == 0) {
         // SwiGLU in the gate_up epilogue: h directly.

@@ -29,3 +29,15 @@ def test_gemm_workspace_holds_smaller_counts(rows, cols):
             assert nbytes >= most[count], count
         else:
             assert nbytes == 0, count
+
+
+@pytest.mark.parametrize("E,k,H,I", [(256, 1, 32, 32), (512, 2, 64, 64), (512, 1, 256, 128), (1024, 8, 64, 32),
+                                     (1024, 2, 128, 64), (8, 2, 1024, 512), (256, 8, 2048, 512)])
+def test_moe_workspace_grows_with_the_tokens(E, k, H, I):
+    """The few-pair tiles' table is longer than a larger call's 80-pair one;
+    at 32 MiB the static scratch's limit decides between the two."""
+    previous = 0
+    for tokens in range(1, min(14 * E // k + 200, 6000)):
+        nbytes = q3x.moe_workspace_bytes(tokens, E, k, H, I)
+        assert nbytes >= previous, tokens
+        previous = nbytes
