@@ -217,7 +217,8 @@ typedef struct q3x_hip_moe_layer_weights {
     int experts, top_k, H, I, shared_I;
 } q3x_hip_moe_layer_weights;
 
-/* Bytes of caller-owned workspace q3x_hip_moe_layer needs for `tokens`. */
+/* Bytes of caller-owned workspace that q3x_hip_moe_layer needs for `tokens` or
+ * fewer tokens: one sized for a caller's most tokens serves every call. */
 size_t q3x_hip_moe_layer_workspace_bytes(const q3x_hip_moe_layer_weights* layer, int tokens);
 
 /* The whole MoE layer for every token t (engine.cpp:406-430; CUDA moe(),

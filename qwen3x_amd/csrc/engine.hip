@@ -1997,15 +1997,9 @@ extern "C" int q3x_hip_engine_create(const q3x_hip_model_config* config, const v
     e->recurrent_floats = static_cast<size_t>(delta_layers) * (conv + memory);
     e->chunk = std::min(context, chunk > 0 ? chunk : kChunk);
     const size_t R = static_cast<size_t>(e->chunk);  // rows of a chunk
-    // The most any row count up to a chunk asks for: a count whose K split
-    // needs partial sums can ask for more than a larger one that has none.
-    // Plans change at multiples of 16 rows only, and between them more rows
-    // ask for more.
+    // Enough for every row count up to a chunk.
     if (c.experts)
-        for (size_t n = 0; n < R + 16; n += 16) {
-            const int count = static_cast<int>(std::min(std::max<size_t>(n, 1), R));
-            e->moe_ws_bytes = std::max(e->moe_ws_bytes, q3x_hip_moe_layer_workspace_bytes(&e->layers[0].moe, count));
-        }
+        e->moe_ws_bytes = q3x_hip_moe_layer_workspace_bytes(&e->layers[0].moe, static_cast<int>(R));
     e->token_capacity = context;
     // The chunked delta rule takes key and value heads of whole 32-wide
     // blocks (every model of the family: 128); others run the token scan.

@@ -1547,7 +1547,19 @@ extern "C" size_t q3x_hip_moe_layer_workspace_bytes(const q3x_hip_moe_layer_weig
     if (!layer || tokens <= 0 || layer->experts <= 0 || layer->top_k <= 0 || layer->H <= 0 || layer->I <= 0 ||
         layer->shared_I <= 0)
         return 0;
-    return moe_layer_layout(tokens, layer->experts, layer->top_k, layer->H, layer->I, layer->shared_I).total;
+    // The most that this or a smaller count needs: a count whose K split needs
+    // partial sums can need more than a larger one that has none (by at most
+    // kPartMost).  The splits change at multiples of 64 tokens, every tile's
+    // height dividing them; between those more tokens need more.
+    constexpr size_t kPartMost = 256u << 20;
+    const auto& w = *layer;
+    size_t most = moe_layer_layout(tokens, w.experts, w.top_k, w.H, w.I, w.shared_I).total;
+    for (int n = (tokens - 1) / 64 * 64; n > 0; n -= 64) {
+        const MoeLayerLayout L = moe_layer_layout(n, w.experts, w.top_k, w.H, w.I, w.shared_I);
+        most = std::max(most, L.total);
+        if (L.total - L.part_bytes + kPartMost < most) break;
+    }
+    return most;
 }
 
 static int moe_layer_checked(const q3x_hip_moe_layer_weights* layer, const float* X, int tokens, float* Y,

@@ -119,8 +119,8 @@ def test_checkpoint_reset_and_errors():
 
 
 def test_moe_prompt_shorter_than_the_chunk():
-    """A MoE layer's workspace does not grow with every token: 256 tokens of
-    this one ask for more than 257 do, and an engine for 257 takes them."""
+    """256 tokens of this MoE layer split K and need more workspace than 257
+    do, and an engine for 257 takes them."""
     _torch()
     fields = dict(CONFIGS["moe_q4"], H=1024, I=512, shared_I=512, VH=8, KH=2, AH=4)
     config, image, _ = synthetic_model(fields, seed=91)

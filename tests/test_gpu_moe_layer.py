@@ -200,3 +200,23 @@ def test_moe_layer_without_routing_outputs_matches_with_them():
         q3x.moe_layer(layer, X, tokens, Y1, ids, wts)
         q3x.moe_layer(layer, X, tokens, Y2)
         assert torch.equal(Y1.view(torch.int32), Y2.view(torch.int32))
+
+
+def test_moe_layer_with_the_workspace_of_more_tokens():
+    """One workspace sized for a caller's most tokens: 256 tokens of this layer
+    split K and need more than 257 do."""
+    torch = _torch()
+    type_, E, H, I, SI, k = Q4_0, 8, 1024, 512, 512, 2
+    rng = np.random.default_rng(8)
+    w = [bf16(rng, E, H, 0.5), random_blocks(rng, type_, E * 2 * I, H), random_blocks(rng, type_, E * H, I),
+         random_blocks(rng, type_, SI, H), random_blocks(rng, type_, SI, H), random_blocks(rng, type_, H, SI),
+         bf16(rng, 1, H, 0.05)]
+    layer = q3x.MoeLayer(*(devb(a) for a in w), type_, E, k, H, I, SI)
+    ws = torch.empty(q3x.moe_layer_workspace_bytes(layer, 257), dtype=torch.uint8, device="cuda:0")
+    for tokens in (257, 256, 65, 64, 2):
+        say(f"moe_layer {tokens} tokens in the workspace of 257")
+        X = dev(rng.normal(0, 1, (tokens, H)).astype(np.float32))
+        Y = [torch.empty((tokens, H), dtype=torch.float32, device="cuda:0") for _ in range(2)]
+        q3x.moe_layer(layer, X, tokens, Y[0], workspace=ws)
+        q3x.moe_layer(layer, X, tokens, Y[1])
+        assert torch.equal(Y[0].view(torch.int32), Y[1].view(torch.int32))

@@ -41,3 +41,14 @@ def test_moe_workspace_grows_with_the_tokens(E, k, H, I):
         nbytes = q3x.moe_workspace_bytes(tokens, E, k, H, I)
         assert nbytes >= previous, tokens
         previous = nbytes
+
+
+@pytest.mark.parametrize("E,k,H,I,SI", [(8, 2, 1024, 512, 512), (8, 2, 1024, 512, 256), (1000, 1, 512, 1728, 1728),
+                                        (64, 8, 1024, 96, 64)])
+def test_moe_layer_workspace_grows_with_the_tokens(E, k, H, I, SI):
+    weights = q3x.MoeLayerWeights(type=Q4_0, experts=E, top_k=k, H=H, I=I, shared_I=SI)
+    previous = 0
+    for tokens in range(1, 700):
+        nbytes = q3x.lib().q3x_hip_moe_layer_workspace_bytes(ctypes.byref(weights), tokens)
+        assert nbytes >= previous, tokens
+        previous = nbytes
