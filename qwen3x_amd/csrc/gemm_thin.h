@@ -177,6 +177,15 @@ __global__ __launch_bounds__(WK * kWave) void gemm_thin_kernel(Policy pol, int r
         first[t] = reinterpret_cast<const uint8_t*>((static_cast<uintptr_t>(hi) << 32) | lo);
         bytes[t] = (max(0, min(16, rows - n)) * row_bytes + 3) & ~3;
     }
+    // Weights pass the caches by, but for a grouped launch's Q8_0 ones on up to
+    // four waves: a segment of 136 bytes shares lines with the next, which a
+    // wave there reads long after (on eight waves another one reads it at the
+    // same time), and an expert's tiles read its rows one after the other.
+    // 19 tokens x top 8 of 256 experts (H 2048, I 512) 125 -> 100 us, 300 321
+    // -> 271, all 300 tokens on the same eight 150 -> 140; Q4_0 (144 bytes) up
+    // to 3% slower cached, eight waves Q8_0 too: 2 tokens x 16 experts, H 16128
+    // 80 us for 74, one matrix 2 x 16 x 65536 51 for 44.
+    constexpr int kPolicy = Policy::kPartialTiles && !U::kQ4 && WK <= 4 ? 0 : kNonTemporal;
     SegRegs<U::WIDE> reg[N];
     auto load_units = [&](int u) {  // past the last unit: zeros, no memory touched
         const bool live = u < units;
@@ -187,8 +196,8 @@ __global__ __launch_bounds__(WK * kWave) void gemm_thin_kernel(Policy pol, int r
                 const_cast<uint8_t*>(first[t] + at), 0, live ? max(0, bytes[t] - at) : 0, kBufferFlags);
 #pragma unroll
             for (int j = 0; j < U::WIDE; ++j)
-                reg[t].wide[j] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[j], 0, kNonTemporal);
-            reg[t].rest = __builtin_amdgcn_raw_buffer_load_b32(rsrc, off[U::WIDE], 0, kNonTemporal);
+                reg[t].wide[j] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off[j], 0, kPolicy);
+            reg[t].rest = __builtin_amdgcn_raw_buffer_load_b32(rsrc, off[U::WIDE], 0, kPolicy);
         }
     };
     auto store_units = [&]() {

@@ -317,12 +317,16 @@ inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 // selected experts get `mean` pairs on average, 0 where the 80-pair tiles
 // are faster: the height that holds the mean and a standard deviation or so,
 // since an expert past it takes a second tile and reads its weights (from the
-// caches) again.  Measured, whole layers, few-pair / 80-pair us: 256 experts
-// top 8, H 2048, I 512, Q4_0: 5 tokens 61 / 96, 19 104 / 159, 64 170 / 277,
-// 180 254 / 314, 300 (11 pairs an expert) 271 / 343; Q8_0 19 148 / 204, 300
-// 362 / 436.  32-row tiles only where few experts leave the 80-pair launch
-// short of workgroups: 8 experts top 8, H 3072, I 1024, Q8_0, 19 tokens 90 /
-// 151, but 32 experts top 2 at 200 tokens 128 / 111.
+// caches) again.  Measured, the routed experts alone, few-pair / 80-pair us
+// (256 experts top 8, H 2048, I 512, even routing): Q4_0 5 tokens 41 / 75, 19
+// 84 / 129, 64 144 / 252, 180 229 / 268, 300 (11 pairs an expert) 236 / 264;
+// Q8_0 43 / 83, 100 / 181, 185 / 333, 251 / 358, 271 / 365.  Routing as 1 /
+// rank gains as much; with all tokens on the same eight experts (few, long
+// groups, cut into many tiles) 64 tokens take 58 / 91, 180 97 / 106 (Q8_0 114
+// / 108), but 300 137 / 109.  The host cannot see the ids, so the height is
+// even routing's.  32-row tiles only where few experts leave the 80-pair launch
+// short of workgroups: whole layers of 8 experts top 8, H 3072, I 1024, Q8_0,
+// 19 tokens 90 / 151, but 32 experts top 2 at 200 tokens 128 / 111.
 inline double moe_live_experts(int tokens, int experts, int top_k) {
     return experts * (1.0 - std::pow(1.0 - static_cast<double>(std::min(top_k, experts)) / experts, tokens));
 }
