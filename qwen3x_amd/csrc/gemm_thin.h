@@ -324,8 +324,8 @@ __global__ __launch_bounds__(WK * kWave) void gemm_thin_kernel(Policy pol, int r
 }
 
 // Waves of a workgroup: eight (two workgroups a CU where the registers
-// allow); four and sixteen measured slower on the 9B's and 27B's matrices
-// except the shortest.
+// allow); four and sixteen measured slower on the 9B's and 27B's matrices but
+// for sixteen on the shortest (1024 rows), where eight are taken too.
 constexpr int kThinWaves = 8;
 constexpr int kThinMaxRows = 32;  // A rows of the largest tile
 
@@ -334,16 +334,20 @@ constexpr int kThinMaxRows = 32;  // A rows of the largest tile
 // (with a K-split workspace) on Q8_0 and Q4_0 matrices of 128 to 20000 rows
 // and 1024 to 24576 columns it took 0.33-0.58 of the time at 2 and 8 tokens,
 // 0.41-0.73 at 16 and 0.45-0.98 at 32 up to 16384 columns; there, past that
-// length, a wave's K units in turn took 0.65 to 1.08 of it.  From 33 tokens
-// on, gemm_x3.h's 64-row tiles read the weights fewer times.
+// length, a wave's K units in turn took 0.65 to 1.08 of it.  (1 to 300 rows of
+// 256 to 65536 columns: 0.53 on average, none slower.)  From 33 tokens on,
+// gemm_x3.h's 64-row tiles read the weights fewer times.
 inline bool thin_ok(int count, int rows, int cols, bool aligned_ok) {
     return aligned_ok && cols <= (1 << 22) && rows <= (1 << 26) && count <= kThinMaxRows && (count <= 16 || cols <= 16384);
 }
 
 // Row tiles per workgroup for `rows` weight rows: as many as leave one
-// workgroup a CU, at most three (more spill registers).  Taller matrices take
-// several workgroups a CU in turn: two row tiles each where the A operand is
-// cheap (at most 8 rows), else three.
+// workgroup a CU, at most three.  Taller matrices take several workgroups a CU
+// in turn: two row tiles each where the A operand is cheap (at most 8 rows),
+// else three.  Registers set the limit: Q8_0 takes 256 for three row tiles of
+// 32 A rows, 246 for 16; Q4_0 on whole units, eight blocks each, is past it
+// from 9 A rows on (16 A rows x 2 and 3 row tiles keep 16 and 92 bytes a lane
+// in scratch, 32 x 3 12), on rows of any length, four blocks a unit, at most 156.
 inline int thin_row_tiles(int rows, int count) {
     const int per_cu = ((rows + 15) / 16 + kCUs - 1) / kCUs;
     return per_cu <= 3 ? per_cu : count <= 8 ? 2 : 3;
@@ -374,7 +378,8 @@ int launch_thin_shape(P pol, int rows, int count, int cols, int tiles_y, hipStre
 
 // One launch over `count` A rows and `rows` weight rows (thin_ok).  7 x 12288
 // x 4096 Q8_0 16 us (43 on gemm_x3.h's tiles; a matvec of it 12), 24 rows 24
-// (45); 7 x 17408 x 5120 Q4_0 25 us (63); 7 x 1024 x 4096 8 us (16).  The A tile is the smallest that holds the rows.
+// (45); 7 x 17408 x 5120 Q4_0 25 us (63); 7 x 1024 x 4096 8 us (16).  The A
+// tile is the smallest that holds the rows.
 template <uint32_t QT, bool ANY, class P>
 int launch_thin_rows(const P& pol, int rows, int count, int cols, hipStream_t stream) {
     // A group of TB blocks must not straddle the row's end.
@@ -396,8 +401,12 @@ int launch_thin(const P& pol, int rows, int count, int cols, bool aligned16, hip
 
 // A grouped launch (a tile table on the device, at most `tiles_y` tiles of
 // `height` rows, about `tiles` of them live): two row tiles a workgroup.  K is
-// split over as many waves as the chip holds at once (16 a CU), no more: a wave
-// waits some microseconds for its first unit whatever follows.
+// split over about 16 waves a CU, no more: a wave waits some microseconds for
+// its first unit whatever follows.  The 4- and 8-row shapes hold 16 at once (12
+// on eight waves in some), the 16- and 32-row ones 8 to 12, but a split for 8
+// there gained nothing (geometric mean 1.00 over 220 calls of 2 to 400 tokens,
+// 0.90 to 1.09).  Two and four waves besides one and eight: 5 tokens x top 4 of
+// 128 experts (H 2048, I 768) Q4_0 34 us for 47, 0.97 over the same calls.
 template <uint32_t QT, bool ANY, class P>
 int launch_thin_grouped(const P& pol, int height, int rows, int cols, int tiles_y, double tiles, hipStream_t stream) {
     using U = SegUnit<QT, ANY>;
