@@ -22,6 +22,11 @@ constexpr int kXcds = 8;  // MI355X: 8 XCDs of 32 CUs
 // none); q3x_hip_gemm_workspace_bytes asks for the smaller counts' too.
 size_t gemm_split_bytes(int rows, int cols, int count);
 
+// The tiles that a GEMM past gemm_thin.h's counts runs on, given `workspace`
+// bytes: {X3Shape, tile rows, tile weight rows, K splits, tiles before the
+// split ones that run whole}.  `paired`: the gate and up launch, over 2 I rows.
+void gemm_plan(int rows, int cols, int count, bool paired, size_t workspace, int plan[5]);
+
 struct GemmTile {
     int m0;      // first A row of the tile (policy-defined numbering)
     int mcount;  // valid A rows in the tile (<= BM)

@@ -120,6 +120,15 @@ size_t gemm_request(int rows, int cols, int count) {
 
 }  // namespace
 
+void q3x::gemm_plan(int rows, int cols, int count, bool paired, size_t workspace, int plan[5]) {
+    const X3Plan p = x3_plan(rows, count, cols, paired, workspace, true);
+    plan[0] = static_cast<int>(p.shape);
+    plan[1] = p.bm;
+    plan[2] = p.bn;
+    plan[3] = p.split;
+    plan[4] = static_cast<int>(p.whole);
+}
+
 size_t q3x::gemm_split_bytes(int rows, int cols, int count) {
     return x3_plan(rows, count, cols, false, SIZE_MAX, true).workspace_bytes();
 }

@@ -47,6 +47,7 @@ def test_gemm_tail_split(type_, rows, cols, count):
 
 
 # The paired gate and up launch: a shared expert of 2 x 8320 rows over 500
-# tokens is 260 tiles, 4 past the CUs.
+# tokens is 260 tiles of 128 x 256, 4 past the CUs.  (test_gpu_gemm_plans.py
+# asserts such a plan for this launch and the tails of the other tiles.)
 def test_paired_tail_split():
     layers.test_moe_layer_parity(Q8_0, 2, 1024, 8448, 8320, 1, 500)

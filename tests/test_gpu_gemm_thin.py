@@ -75,6 +75,25 @@ def test_few_token_gemm_keeps_tokens_apart(type_, tokens):
 
 
 @pytest.mark.parametrize("type_", [Q8_0, Q4_0])
+@pytest.mark.parametrize("cols", [96, 1056, 4128])
+def test_few_token_gemm_keeps_tokens_apart_at_the_row_end(type_, cols):
+    """The same where K ends in a short unit: its registers also hold the next
+    row's first blocks and the last block's activations again."""
+    rows, tokens = 47, 7
+    rng = np.random.default_rng(cols)
+    w = random_blocks(rng, type_, rows, cols)
+    X = rng.normal(0, 1, (tokens, cols)).astype(np.float32)
+    clean = _run(type_, w, rows, cols, X, 0, False)
+    for col in (0, cols - 33, cols - 32, cols - 1):
+        bad = X.copy()
+        bad[1, col] = np.inf
+        got = _run(type_, w, rows, cols, bad, 0, False)
+        keep = [t for t in range(tokens) if t != 1]
+        assert np.array_equal(got[keep], clean[keep])
+        assert not np.isfinite(got[1]).any()
+
+
+@pytest.mark.parametrize("type_", [Q8_0, Q4_0])
 @pytest.mark.parametrize("E,k,tokens", [(16, 2, 2), (16, 2, 4), (8, 2, 12), (4, 2, 20), (4, 2, 40), (300, 1, 5)])
 @pytest.mark.parametrize("H,I", [(256, 256), (288, 96), (320, 160), (1056, 32)])
 def test_few_pair_experts(type_, E, k, tokens, H, I):
