@@ -57,6 +57,8 @@
 // and a wave skips the subtile rows past the valid ones.
 #pragma once
 
+#include <algorithm>
+
 #include "gemm.h"
 
 namespace q3x {
@@ -598,6 +600,11 @@ inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspa
         const long long t = tiles(o.bm, o.bn);
         const double area = static_cast<double>(o.bm) * o.bn;
         const double unit = 2.0 * cols * kCUs / 1e12;  // seconds of area / rate
+        // No split of the shape takes less than its tiles evenly spread at its
+        // best rate (rounded down), and none less than that and its fixup.
+        const double least = static_cast<double>(t) / kCUs * area * unit * (1.0 - 1e-9) /
+                             *std::max_element(o.rate, o.rate + o.occupancy);
+        if (least > best_t) continue;
         // The tiles of the full rounds, where a short round follows them: the
         // one-per-CU shapes may split that round's tiles alone, to at most
         // two units per CU (64 MiB of sums).  Measured with the best plan
@@ -608,9 +615,12 @@ inline X3Plan x3_plan(int rows, int count, int cols, bool paired, size_t workspa
         // tokens x 4096 to 24576 rows no choice was slower than before.
         const long long rounds = t / kCUs * kCUs;
         const bool tail = o.occupancy == 1 && rounds > 0 && rounds < t;
-        for (const long long whole : {0LL, tail ? rounds : 0LL}) {
-            const long long part = t - whole;
+        for (int tailed = 0; tailed <= tail; ++tailed) {
+            const long long whole = tailed ? rounds : 0, part = t - whole;
             for (const int split : kSplits) {
+                const double fixup =
+                    split > 1 ? kLaunchSeconds + static_cast<double>(part) * area * 4.0 * (split + 1) / fixup_rate : 0.0;
+                if (least + fixup * (1.0 - 1e-9) > best_t) break;
                 const int per = (blocks + split - 1) / split;
                 if (split > 1 && (per < (o.shape == X3Shape::k64x128_split ? 16 : 8) || (split - 1) * per >= blocks)) continue;
                 if (whole > 0 ? split == 1 || part * split > kTailUnits : split > o.most_split) continue;
