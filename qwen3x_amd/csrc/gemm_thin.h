@@ -177,15 +177,18 @@ __global__ __launch_bounds__(WK * kWave) void gemm_thin_kernel(Policy pol, int r
         first[t] = reinterpret_cast<const uint8_t*>((static_cast<uintptr_t>(hi) << 32) | lo);
         bytes[t] = (max(0, min(16, rows - n)) * row_bytes + 3) & ~3;
     }
-    // Weights pass the caches by, but for a grouped launch's Q8_0 ones on up to
-    // four waves: a segment of 136 bytes shares lines with the next, which a
-    // wave there reads long after (on eight waves another one reads it at the
-    // same time), and an expert's tiles read its rows one after the other.
-    // 19 tokens x top 8 of 256 experts (H 2048, I 512) 125 -> 100 us, 300 321
-    // -> 271, all 300 tokens on the same eight 150 -> 140; Q4_0 (144 bytes) up
-    // to 3% slower cached, eight waves Q8_0 too: 2 tokens x 16 experts, H 16128
-    // 80 us for 74, one matrix 2 x 16 x 65536 51 for 44.
-    constexpr int kPolicy = Policy::kPartialTiles && !U::kQ4 && WK <= 4 ? 0 : kNonTemporal;
+    // Weights pass the caches by, but for a grouped launch's Q8_0 ones on one or
+    // two waves (many tiles): a segment of 136 bytes shares lines with the
+    // next, which a wave there reads long after (on more waves another one reads
+    // it at the same time), and an expert's tiles read its rows one after the
+    // other.  19 tokens x top 8 of 256 experts (H 2048, I 512) 125 -> 100 us,
+    // 300 321 -> 271, all 300 tokens on the same eight 150 -> 143; 300 drawn
+    // layers, their weights in turn from memory, 0.98 (0.78 to 0.9 where the
+    // experts hold some 500 MB, 1.03 for 101 tokens top 4 of 256, H 1280, I
+    // 128).  Q4_0 (144 bytes) up to 3% slower cached, Q8_0 on four waves up to 4%
+    // (20 tokens top 2 of 32, H 1792, I 736), on eight 9% (2 tokens top 1 of 16,
+    // H 16128), one matrix 2 x 16 x 65536 51 us for 44.
+    constexpr int kPolicy = Policy::kPartialTiles && !U::kQ4 && WK <= 2 ? 0 : kNonTemporal;
     SegRegs<U::WIDE> reg[N];
     auto load_units = [&](int u) {  // past the last unit: zeros, no memory touched
         const bool live = u < units;
